@@ -14,9 +14,11 @@
 // counter for the other splits, sums the group's partials in split order
 // (deterministic, no atomics on data) and contracts the state with the
 // split's relu(q) on MFMA.  Counters live in the workspace's control words.
-// Other head dims (128 % D == 0) and fp32 input take a VALU path in three
-// launches (split states, fixed-order split reduction, output).
-#include "kf_common.h"
+// Other head dims (128 % D == 0) and fp32 input take three launches (split
+// states, fixed-order split reduction, output): on the matrix cores from
+// D = 16 (linattn_wide.h), on the VALU for D = 1..8 and for buffers that are
+// not 16-byte aligned.
+#include "linattn_wide.h"
 
 #include <atomic>
 #include <mutex>
@@ -838,6 +840,7 @@ struct Launch {
     int spin_limit;
     bool force_ticket;     // number workgroups by ticket even when all fit at once
     bool out_tn;           // out[b][c][t] instead of out[b][t][c]
+    bool wide;             // buffers the matrix-core kernels of linattn_wide.h can read
     hipStream_t stream;
 };
 
@@ -907,8 +910,49 @@ int run_mfma(const Launch& a) {
     return KF_OK;
 }
 
+// Head groups of one linattn_wide.h launch: heads sharing a workgroup's 64
+// (D = 128: 128) channels.
+int64_t wide_groups(int64_t heads, int64_t dim) {
+    const int64_t hg = dim >= 64 ? 1 : 64 / dim;
+    return (heads + hg - 1) / hg;
+}
+
+template <typename T, typename TO, int DG>
+int run_wide(const Launch& a) {
+    const int ng = (int)wide_groups(a.H, DG), groups = a.B * ng;
+    hipLaunchKernelGGL((linattn_wide_state_kernel<T, DG>), dim3(groups, a.S), dim3(kWideThreads), 0, a.stream,
+                       static_cast<const T*>(a.qkv), a.ws.partial, a.N, a.H, ng, a.L, a.S);
+    if (int rc = check_launch("linattn_wide_state_kernel launch")) return rc;
+    if (int rc = launch_reduce(a.ws.partial, a.ws.state, (int64_t)a.B * a.H, a.S, (DG + 1) * DG, a.stream))
+        return rc;
+    // Runs of whole 128-token tiles, as many as keep the launch within one
+    // round of resident workgroups, so that a workgroup's state rows serve
+    // several tiles and no partial round is left.
+    int64_t runs = 2 * (int64_t)device_cu_count() / groups;
+    if (runs < 1) runs = 1;
+    const int64_t tiles = (a.N + kTT - 1) / kTT;
+    if (runs > tiles) runs = tiles;
+    const int run_len = (int)((tiles + runs - 1) / runs) * kTT;
+    const dim3 grid(groups, (a.N + run_len - 1) / run_len);
+    if constexpr (sizeof(TO) == 4) {
+        if (a.out_tn) {
+            hipLaunchKernelGGL((linattn_wide_out_kernel<T, TO, DG, true>), grid, dim3(kWideThreads), 0, a.stream,
+                               static_cast<const T*>(a.qkv), a.ws.state, static_cast<TO*>(a.out), a.N, a.H, ng,
+                               run_len, a.eps);
+            return check_launch("linattn_wide_out_kernel launch");
+        }
+    }
+    hipLaunchKernelGGL((linattn_wide_out_kernel<T, TO, DG, false>), grid, dim3(kWideThreads), 0, a.stream,
+                       static_cast<const T*>(a.qkv), a.ws.state, static_cast<TO*>(a.out), a.N, a.H, ng, run_len,
+                       a.eps);
+    return check_launch("linattn_wide_out_kernel launch");
+}
+
 template <typename T, typename TO, int DG>
 int run_generic(const Launch& a) {
+    if constexpr (DG >= 16 && !(DG == kD && sizeof(T) == 2)) {
+        if (a.wide) return run_wide<T, TO, DG>(a);
+    }
     hipLaunchKernelGGL((linattn_state_generic<T, DG>), dim3(a.H, a.S, a.B), dim3(256), 0, a.stream,
                        static_cast<const T*>(a.qkv), a.ws.partial, a.N, a.H, a.L, a.S);
     if (int rc = check_launch("linattn_state_generic launch")) return rc;
@@ -1040,6 +1084,11 @@ int linattn_run(const void* qkv, void* out, void* workspace, int64_t workspace_b
     a.spin_limit = spin_limit;
     a.force_ticket = force_ticket;
     a.out_tn = out_tn;
+    // linattn_wide.h reads and writes whole 16-byte chunks (rows are whole
+    // chunks from D = 16); its grids count a 512-thread workgroup per head
+    // group in x, which HIP limits to 2^32 threads.
+    a.wide = (uintptr_t)qkv % 16 == 0 && (uintptr_t)out % 16 == 0 && dim >= 16 &&
+             batch * wide_groups(heads, dim) < (1 << 22) && (!out_tn || out_dtype == KF_F32);
     a.stream = s;
     switch (in_dtype) {
         case KF_BF16: return run_in<bf16>(out_dtype, mfma, a);
@@ -1124,7 +1173,8 @@ extern "C" int64_t kf_linattn_default_splits(int64_t batch, int64_t heads, int64
     // some CUs with two workgroups and others with one ran 10-20% slower on
     // MI355X than one workgroup per CU (B=2, H=70, N=4096: 36.3 us at 3 splits
     // = 210 workgroups, 41.8 us at 4 = 280; B=1, N=16384: 57.6 us at 7 = 245,
-    // 74.1 us at 8 = 280).  Other head dims: about 1.75 workgroups per CU.
+    // 74.1 us at 8 = 280).  Other head dims: about 1.75 workgroups per CU (one
+    // per head group of linattn_wide.h from D = 16, one per head below).
     if (batch <= 0 || heads <= 0 || seq_len <= 0) return 1;
     const int64_t cus = kf::device_cu_count();
     int64_t splits;
@@ -1132,7 +1182,7 @@ extern "C" int64_t kf_linattn_default_splits(int64_t batch, int64_t heads, int64
         const int64_t groups = batch * ((heads + 1) / 2);
         splits = cus / groups;
     } else {
-        const int64_t groups = batch * heads;
+        const int64_t groups = batch * (dim == 16 ? kf::wide_groups(heads, dim) : heads);
         splits = ((7 * cus + 3) / 4 + groups - 1) / groups;
     }
     const int64_t max_splits = (seq_len + kf::kTT - 1) / kf::kTT;
