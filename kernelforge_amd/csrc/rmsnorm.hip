@@ -49,6 +49,31 @@ __device__ __forceinline__ void store_nt(Pack<T, N>* dst, const Pack<T, N>& p) {
     }
 }
 
+// Non-temporal load of a Pack of 8, 16 or 32 bytes.
+template <typename T, int N>
+__device__ __forceinline__ Pack<T, N> load_nt(const Pack<T, N>* src) {
+    constexpr int BYTES = sizeof(T) * N;
+    Pack<T, N> p;
+    if constexpr (BYTES % 16 == 0) {
+        u32x4* d = reinterpret_cast<u32x4*>(&p);
+#pragma unroll
+        for (int i = 0; i < BYTES / 16; ++i) d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src) + i);
+    } else {
+        static_assert(BYTES == 8, "packs are 8, 16 or 32 bytes");
+        *reinterpret_cast<u32x2*>(&p) = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(src));
+    }
+    return p;
+}
+
+// Workgroup barrier that waits for LDS traffic only and leaves global loads
+// in flight.
+__device__ __forceinline__ void barrier_lds_only() {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt untouched
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // x and y rows start every ld_x / ld_y elements (ld >= dim); the vector path
 // needs those strides, like the base pointers, aligned to the vector slices.
 // y may alias x (in place, same stride and type): every row is read whole
@@ -227,10 +252,167 @@ int dispatch(const void* x, const void* w, void* y, int64_t rows, int64_t dim, i
 //   dx  = inv * g - x * inv^3 * sum(g * x) / dim
 //   dw  = tw(sum over rows of float(dy) * float(n))   (fp32 sum of unrounded
 //                                               products)
-// Each block owns a contiguous run of rows and keeps its dw partial sums in
-// fp32 in `partial[block][dim]` (its own row of the workspace, so no two
+// Each block owns a contiguous run of rows and writes its dw partial sums in
+// fp32 to `partial[block][dim]` (its own row of the workspace, so no two
 // blocks touch the same partial); rmsnorm_dw_reduce_kernel then adds the
-// block partials in block order (fixed order: deterministic, no atomics).
+// block partials in a fixed order (deterministic, no atomics).
+
+// Rows of whole 16-byte vectors, laid out over the lanes as in
+// rmsnorm_vec_kernel (RPB = WAVES / WPR rows at a time).  x and dy are read
+// once, dx written once: HBM bound.  Every lane owns the same columns of all
+// its rows, so the weight and the dw sums stay in registers; the next row's
+// loads run while this row is reduced.  Measured on MI355X at rows 8192, dim
+// 2240, bf16 x, fp32 weight (147 MB): 38 us, 3.9 TB/s;
+// one scalar load at a time, with the dw sums read and written in memory for
+// every row, took 87.
+template <typename TX, typename TW, typename TY, int VPT, int WPR, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rmsnorm_bwd_vec_kernel(const TX* __restrict__ x,
+                                                                     const TW* __restrict__ w,
+                                                                     const TY* __restrict__ dy,
+                                                                     TX* __restrict__ dx,
+                                                                     float* __restrict__ partial, int64_t rows,
+                                                                     int dim, int64_t rows_per_block, float eps) {
+    constexpr int VEC = 16 / sizeof(TX);
+    typedef Pack<TW, VEC> WPack;
+    typedef Pack<TY, VEC> YPack;
+    constexpr int RPB = WAVES / WPR;
+    constexpr int SLOTS = VPT * WPR * 64;
+    constexpr bool kAhead = VPT <= 2;  // registers for a second row
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int slot = wave / WPR, slice = wave % WPR;
+    const int nvec = dim / VEC;
+    const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
+    const int64_t r1 = r0 + rows_per_block < rows ? r0 + rows_per_block : rows;
+
+    WPack wv[VPT];
+    float acc[VPT][VEC];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int j = (i * WPR + slice) * 64 + lane;
+        wv[i] = reinterpret_cast<const WPack*>(w)[j < nvec ? j : 0];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[i][k] = 0.f;
+    }
+    // One row of x and dy; a row past the run re-reads its last row, and a
+    // vector past the row's end is left zero.
+    auto load = [&](int64_t row, u32x4 (&xv)[VPT], YPack (&gv)[VPT]) {
+        if (row >= r1) row = r1 - 1;
+        const u32x4* xr = reinterpret_cast<const u32x4*>(x + row * dim);
+        const YPack* gr = reinterpret_cast<const YPack*>(dy + row * dim);
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const int j = (i * WPR + slice) * 64 + lane;
+            if (j < nvec) {
+                xv[i] = __builtin_nontemporal_load(xr + j);
+                gv[i] = load_nt(gr + j);
+            } else {
+                xv[i] = u32x4{0u, 0u, 0u, 0u};
+                gv[i] = YPack{};
+            }
+        }
+    };
+    u32x4 xv[VPT], xn[VPT];
+    YPack gv[VPT], gn[VPT];
+    load(r0 + slot, xv, gv);
+    __shared__ float part[2][WAVES][2];
+    const int64_t steps = (r1 - r0 + RPB - 1) / RPB;
+    for (int64_t it = 0; it < steps; ++it) {
+        const int64_t row = r0 + it * RPB + slot;
+        if constexpr (kAhead) load(row + RPB, xn, gn);
+        float ss = 0.f, dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const TX* e = reinterpret_cast<const TX*>(&xv[i]);
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                const float f = to_f32(e[k]);
+                const float g = to_f32(from_f32<TX>(to_f32(gv[i].v[k]) * to_f32(wv[i].v[k])));
+                ss = fmaf(f, f, ss);
+                dot = fmaf(g, f, dot);
+            }
+        }
+        ss = wave_sum(ss);
+        dot = wave_sum(dot);
+        if constexpr (WPR > 1) {
+            // Two sets of slots in turn: one barrier per row, which leaves the
+            // next row's loads in flight.
+            float (*pt)[2] = part[it & 1];
+            if (lane == 0) {
+                pt[wave][0] = ss;
+                pt[wave][1] = dot;
+            }
+            barrier_lds_only();
+            ss = dot = 0.f;
+#pragma unroll
+            for (int q = 0; q < WPR; ++q) {
+                ss += pt[slot * WPR + q][0];
+                dot += pt[slot * WPR + q][1];
+            }
+        }
+        const float inv = 1.0f / sqrtf(ss / (float)dim + eps);
+        const float kk = inv * inv * inv * dot / (float)dim;
+        if (row < r1) {
+            u32x4* dr = reinterpret_cast<u32x4*>(dx + row * dim);
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) {
+                const int j = (i * WPR + slice) * 64 + lane;
+                const TX* e = reinterpret_cast<const TX*>(&xv[i]);
+                u32x4 ov;
+                TX* o = reinterpret_cast<TX*>(&ov);
+#pragma unroll
+                for (int k = 0; k < VEC; ++k) {
+                    const float f = to_f32(e[k]);
+                    const float gy = to_f32(gv[i].v[k]);
+                    const float g = to_f32(from_f32<TX>(gy * to_f32(wv[i].v[k])));
+                    o[k] = from_f32<TX>(inv * g - f * kk);
+                    if (j < nvec) acc[i][k] += gy * to_f32(from_f32<TX>(f * inv));
+                }
+                if (j < nvec) __builtin_nontemporal_store(ov, dr + j);
+            }
+        }
+        if constexpr (kAhead) {
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) {
+                xv[i] = xn[i];
+                gv[i] = gn[i];
+            }
+        } else {
+            load(row + RPB, xv, gv);
+        }
+    }
+    // The row slots' sums in slot order.
+    if constexpr (RPB > 1) {
+        __shared__ float comb[(RPB - 1) * SLOTS * VEC];
+        if (slot > 0) {
+#pragma unroll
+            for (int i = 0; i < VPT; ++i)
+#pragma unroll
+                for (int k = 0; k < VEC; ++k)
+                    comb[((slot - 1) * VEC + k) * SLOTS + (i * WPR + slice) * 64 + lane] = acc[i][k];
+        }
+        __syncthreads();
+        if (slot > 0) return;
+#pragma unroll
+        for (int q = 0; q < RPB - 1; ++q)
+#pragma unroll
+            for (int i = 0; i < VPT; ++i)
+#pragma unroll
+                for (int k = 0; k < VEC; ++k)
+                    acc[i][k] += comb[(q * VEC + k) * SLOTS + (i * WPR + slice) * 64 + lane];
+    }
+    f32x4* pw = reinterpret_cast<f32x4*>(partial + (int64_t)blockIdx.x * dim);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int j = (i * WPR + slice) * 64 + lane;
+        if (j < nvec) {
+#pragma unroll
+            for (int k = 0; k < VEC; k += 4)
+                pw[(j * VEC + k) / 4] = f32x4{acc[i][k], acc[i][k + 1], acc[i][k + 2], acc[i][k + 3]};
+        }
+    }
+}
+
+// Any dim / alignment: a block's rows one after another, two passes over each.
 template <typename TX, typename TW, typename TY>
 __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const TX* __restrict__ x,
                                                              const TW* __restrict__ w,
@@ -279,36 +461,108 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const TX* __restric
     }
 }
 
+// dw = the block partials' sums: 32 columns per block, 16 slices of the
+// partials each (slice s adds partials s, s + 16, ..., eight loads in flight),
+// then the slices in order.  One thread per column over all partials was a
+// chain of up to 1024 load latencies (227 us at 1024 partials of 2240 columns
+// on MI355X; now 4.8).
+constexpr int kDwCols = 32, kDwSlices = 16;
 template <typename TW>
-__global__ __launch_bounds__(kBlock) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial,
-                                                                   TW* __restrict__ dw, int64_t dim,
-                                                                   int nblocks) {
-    const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (c >= dim) return;
+__global__ __launch_bounds__(kDwCols * kDwSlices) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial,
+                                                                                 TW* __restrict__ dw, int64_t dim,
+                                                                                 int nblocks) {
+    __shared__ float sums[kDwSlices][kDwCols];
+    const int col = threadIdx.x % kDwCols, slice = threadIdx.x / kDwCols;
+    const int64_t c = (int64_t)blockIdx.x * kDwCols + col;
     float acc = 0.f;
-    for (int b = 0; b < nblocks; ++b) acc += partial[(int64_t)b * dim + c];
-    dw[c] = from_f32<TW>(acc);
+    if (c < dim) {
+        for (int b0 = slice; b0 < nblocks; b0 += 8 * kDwSlices) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int b = b0 + i * kDwSlices;
+                const float p = partial[(int64_t)(b < nblocks ? b : b0) * dim + c];
+                v[i] = b < nblocks ? p : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc += v[i];
+        }
+    }
+    sums[slice][col] = acc;
+    __syncthreads();
+    if (slice == 0 && c < dim) {
+#pragma unroll
+        for (int q = 1; q < kDwSlices; ++q) acc += sums[q][col];
+        dw[c] = from_f32<TW>(acc);
+    }
 }
 
-constexpr int64_t kBwdMaxBlocks = 1024;
+constexpr int64_t kBwdMaxBlocks = 1024;  // partials of the workspace
 
 int64_t bwd_blocks(int64_t rows) { return rows < kBwdMaxBlocks ? rows : kBwdMaxBlocks; }
+
+template <typename TX, typename TW, typename TY, int VPT, int WPR, int WAVES>
+int launch_bwd_vec(const TX* x, const TW* w, const TY* dy, TX* dx, float* partial, int64_t rows, int64_t dim,
+                   float eps, hipStream_t stream, int64_t* used) {
+    // As many blocks as stay resident: 16 wavefronts per CU for fp32 x, 8 for
+    // 16-bit x, whose kernels take 120-140 registers (rows 16384, dim 4096 on
+    // MI355X: bf16 x, fp32 weight 116 us at 16, 102 at 8; fp32 150 and 167),
+    // each with at least four rounds of rows where the rows allow it (a
+    // block's partial costs two extra passes over a row's width).
+    constexpr int RPB = WAVES / WPR;
+    constexpr int kWavesPerCu = sizeof(TX) == 4 ? 16 : 8;
+    int64_t nb = (int64_t)device_cu_count() * (kWavesPerCu / WAVES);
+    const int64_t by_rows = (rows + 4 * RPB - 1) / (4 * RPB);
+    if (nb > by_rows) nb = by_rows;
+    if (nb > bwd_blocks(rows)) nb = bwd_blocks(rows);
+    const int64_t per = (rows + nb - 1) / nb;
+    *used = (rows + per - 1) / per;
+    hipLaunchKernelGGL((rmsnorm_bwd_vec_kernel<TX, TW, TY, VPT, WPR, WAVES>), dim3((unsigned)*used),
+                       dim3(64 * WAVES), 0, stream, x, w, dy, dx, partial, rows, (int)dim, per, eps);
+    return check_launch("rmsnorm_bwd_vec_kernel launch");
+}
+
+template <typename TX, typename TW, typename TY>
+int run_bwd_rows(const TX* x, const TW* w, const TY* dy, TX* dx, float* partial, int64_t rows, int64_t dim,
+                 float eps, hipStream_t stream, int64_t* used) {
+    constexpr int VEC = 16 / sizeof(TX);
+    constexpr size_t WA = sizeof(Pack<TW, VEC>) < 16 ? sizeof(Pack<TW, VEC>) : 16;
+    constexpr size_t YA = sizeof(Pack<TY, VEC>) < 16 ? sizeof(Pack<TY, VEC>) : 16;
+    const bool aligned = aligned_to(x, 16) && aligned_to(dx, 16) && aligned_to(dy, YA) && aligned_to(w, WA) &&
+                         aligned_to(partial, 16) && dim % VEC == 0;
+    const int64_t nvec = dim / VEC;
+    if (aligned) {
+#define KF_RMS_BWD(VPT, WPR, WAVES) \
+    return launch_bwd_vec<TX, TW, TY, VPT, WPR, WAVES>(x, w, dy, dx, partial, rows, dim, eps, stream, used)
+        // (vectors per lane, waves per row, waves per block).
+        if (nvec <= 64) KF_RMS_BWD(1, 1, 4);
+        if (nvec <= 128) KF_RMS_BWD(2, 1, 4);
+        if (nvec <= 256) KF_RMS_BWD(2, 2, 4);
+        if (nvec <= 512) KF_RMS_BWD(2, 4, 4);
+        if (nvec <= 1024) KF_RMS_BWD(2, 8, 8);
+        if (nvec <= 2048) KF_RMS_BWD(4, 8, 8);
+#undef KF_RMS_BWD
+    }
+    const int64_t nb = bwd_blocks(rows);
+    const int64_t per = (rows + nb - 1) / nb;
+    *used = (rows + per - 1) / per;  // blocks that own at least one row
+    hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TY>), dim3((unsigned)*used), dim3(kBlock), 0, stream, x, w, dy,
+                       dx, partial, rows, dim, per, eps);
+    return check_launch("rmsnorm_bwd_kernel launch");
+}
 
 template <typename TX, typename TW, typename TY>
 int run_bwd(const void* x, const void* w, const void* dy, void* dx, void* dw, float* partial,
             int64_t rows, int64_t dim, float eps, hipStream_t stream) {
-    const int64_t nb = bwd_blocks(rows);
-    const int64_t per = nb > 0 ? (rows + nb - 1) / nb : 1;
-    const int64_t used = (rows + per - 1) / per;  // blocks that own at least one row
-    if (used > 0) {
-        hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TY>), dim3((unsigned)used), dim3(kBlock), 0, stream,
-                           static_cast<const TX*>(x), static_cast<const TW*>(w), static_cast<const TY*>(dy),
-                           static_cast<TX*>(dx), partial, rows, dim, per, eps);
-        if (int rc = check_launch("rmsnorm_bwd_kernel launch")) return rc;
+    int64_t used = 0;
+    if (rows > 0) {
+        if (int rc = run_bwd_rows(static_cast<const TX*>(x), static_cast<const TW*>(w), static_cast<const TY*>(dy),
+                                  static_cast<TX*>(dx), partial, rows, dim, eps, stream, &used))
+            return rc;
     }
     // With no rows the reduction adds nothing and writes a zero weight gradient.
-    hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<TW>), dim3((unsigned)((dim + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, stream, partial, static_cast<TW*>(dw), dim, (int)used);
+    hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<TW>), dim3((unsigned)((dim + kDwCols - 1) / kDwCols)),
+                       dim3(kDwCols * kDwSlices), 0, stream, partial, static_cast<TW*>(dw), dim, (int)used);
     return check_launch("rmsnorm_dw_reduce_kernel launch");
 }
 
