@@ -354,6 +354,20 @@ int kf_fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
               int64_t D, float scale, int causal, int dtype, kf_stream_t stream);
 
 /*
+ * The same with a workspace, which lets small grids (short sequences, few
+ * heads, decoding) split each tile's keys over several workgroups.
+ * kf_fa_fwd_workspace_bytes gives the bytes the shape's split takes (0: none
+ * needed, negative: unsupported shape); the workspace must be 16-byte aligned
+ * and needs no initialisation.  With less, or none, the call runs as kf_fa_fwd.
+ */
+int64_t kf_fa_fwd_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                                  int causal);
+int kf_fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                 void* workspace, int64_t workspace_bytes,
+                 int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                 float scale, int causal, int dtype, kf_stream_t stream);
+
+/*
  * tO from the cached LSE (standalone JVP, no forward launch):
  *   P = exp(scale*q k^T - lse),  tS = scale*(tq k^T + q tk^T),  H = P*tS,
  *   tO = P tv + H v - rowsum(H) * O.
@@ -387,6 +401,15 @@ int kf_fa_fwd_jvp(const void* q, const void* k, const void* v,
                   int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
                   int64_t D, float scale, int causal, int dtype,
                   kf_stream_t stream);
+
+/* The same with a workspace (see kf_fa_fwd_ws). */
+int64_t kf_fa_fwd_jvp_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                                      int causal);
+int kf_fa_fwd_jvp_ws(const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                     const void* tv, void* o, float* lse, void* to,
+                     void* workspace, int64_t workspace_bytes,
+                     int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                     float scale, int causal, int dtype, kf_stream_t stream);
 
 /*
  * Workspace bytes kf_fa_bwd needs (fp32 per-row statistics, rows padded to

@@ -71,6 +71,12 @@ SIGNATURES = {
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
          _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
     ),
+    "kf_fa_fwd_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
+    "kf_fa_fwd_ws": (
+        _int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64,
+         _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
+    ),
     "kf_fa_jvp": (
         _int,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
@@ -82,6 +88,12 @@ SIGNATURES = {
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
          _c_void_p, _c_void_p, _c_void_p,
          _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
+    ),
+    "kf_fa_fwd_jvp_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
+    "kf_fa_fwd_jvp_ws": (
+        _int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
     ),
     "kf_fa_bwd_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
     "kf_fa_bwd": (
@@ -109,6 +121,11 @@ MEASURE_SIGNATURES = {
          _c_void_p],
     ),
     "kfm_linattn_split_plan": (_int, [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
+    "kfm_fa_fwd_split": (
+        _int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _int, _int, _c_void_p],
+    ),
     "kfm_fa_bwd_blocks": (
         _int,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,

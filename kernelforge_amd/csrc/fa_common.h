@@ -94,6 +94,12 @@ struct FaParams {
     float scale;       // natural units
     float scale_log2;  // scale * log2(e)
     int causal;
+    // Split forward modes (fa_split_kernel) only.
+    int splits;        // key ranges per query tile
+    int pack;          // rows of a tile: 1 = (query, head of the KV head's group) pairs, 0 = queries of one head
+    float* ws_u;       // [splits][B * Hq * Nq][D] unnormalised outputs U (splits > 1)
+    float* ws_g;       // the same of G (FWD_JVP)
+    float* ws_st;      // [splits][B * Hq * Nq][4]: exponent reference (log2), fp32 row sum, l, r
 };
 
 // Physical 16-byte chunk = logical chunk ^ swz(row), for CH chunks per row.

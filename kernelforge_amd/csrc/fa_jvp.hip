@@ -76,6 +76,35 @@ __device__ __forceinline__ FaBlock fa_block(const FaParams& p) {
     return r;
 }
 
+// The split forward's workgroup: a query tile, a head (KV head when rows are
+// packed), a batch and a key range.  Tiles of one key range follow one another
+// (they share its K and V in an XCD's L2); under a causal mask every head's
+// longest tile starts before any shorter one instead.
+struct FaSplitBlock {
+    int qtile, h, b, s;
+};
+__device__ __forceinline__ FaSplitBlock fa_split_block(const FaParams& p) {
+    const int nblk = gridDim.x, id = blockIdx.x;
+    const int heads = p.pack ? p.Hkv : p.Hq;
+    FaSplitBlock r;
+    int rest;
+    if (p.causal) {
+        const int per_tile = nblk / p.n_qtiles;
+        r.qtile = p.n_qtiles - 1 - id / per_tile;
+        rest = id % per_tile;
+    } else {
+        const int per = nblk >> 3, rem = nblk & 7, xcd = id & 7, slot = id >> 3;
+        const int lg = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+        r.qtile = lg % p.n_qtiles;
+        rest = lg / p.n_qtiles;
+    }
+    r.s = rest % p.splits;
+    rest /= p.splits;
+    r.h = rest % heads;
+    r.b = rest / heads;
+    return r;
+}
+
 // Row blocks of 16 query rows per wavefront.  The forward has the registers
 // for two (a 256-row workgroup): every K row and V^T operand read from LDS
 // then feeds two MFMAs, and a tile copy serves twice the rows.
@@ -92,11 +121,14 @@ template <int DP, int MODE> constexpr int fa_rows() { return FaTile<DP>::BQ * fa
 // products): a workgroup with a row past kCachedOBound writes NaN into the
 // first tO element of its first row (and nothing else), and fa_fixup_kernel
 // redoes its rows with LAZY = true, the scan that recomputes U.  kbuf0/1 and
-// vbuf0/1 are the two K-side and V-side LDS buffers, NT tiles each.
-template <typename T, int DP, int MODE, bool ALL, bool LAZY>
+// vbuf0/1 are the two K-side and V-side LDS buffers, NT tiles each.  SPLIT
+// (FWD and FWD_JVP with LAZY = true): the workgroup scans one of p.splits key
+// ranges of its tile (fa_split_kernel).
+template <typename T, int DP, int MODE, bool ALL, bool LAZY, bool SPLIT = false>
 __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T* vbuf0, T* vbuf1) {
-    constexpr int R = fa_row_blocks<DP, MODE>();
-    constexpr int kBQ = fa_rows<DP, MODE>(), kBK = FaTile<DP>::BK;
+    static_assert(!SPLIT || (MODE != FA_JVP && LAZY), "the split scan is the rescaling one");
+    constexpr int R = SPLIT ? 1 : fa_row_blocks<DP, MODE>();
+    constexpr int kBQ = FaTile<DP>::BQ * R, kBK = FaTile<DP>::BK;
     constexpr bool JVP = MODE != FA_FWD;
     constexpr bool kCachedO = MODE == FA_JVP && !LAZY;  // O from p.o, no U products
     constexpr int NT = JVP ? 2 : 1;   // tensors per side: K (, tK) and V (, tV)
@@ -123,9 +155,24 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = lane >> 4;  // 16-lane group: key sub-range / d sub-range
 
-    const FaBlock blk = fa_block(p);
-    const int qtile = blk.qtile, hq = blk.hq, b = blk.b;
-    const int hk = hq / p.group;
+    int qtile, hq, b, hk, split = 0;
+    // Packed rows: row r is query r / group of head hk * group + r % group.
+    int group = 1;
+    if constexpr (SPLIT) {
+        const FaSplitBlock blk = fa_split_block(p);
+        qtile = blk.qtile;
+        b = blk.b;
+        split = blk.s;
+        if (p.pack) group = p.group;
+        hk = p.pack ? blk.h : blk.h / p.group;
+        hq = p.pack ? blk.h * p.group : blk.h;
+    } else {
+        const FaBlock blk = fa_block(p);
+        qtile = blk.qtile;
+        hq = blk.hq;
+        b = blk.b;
+        hk = hq / p.group;
+    }
 
     const int q0w = qtile * kBQ + wave * 16 * R;  // first row of this wavefront
     const int64_t q_row_stride = (int64_t)p.Hq * p.D;
@@ -136,11 +183,16 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
     int qr[R];
     bool row_ok[R];
     int64_t q_off[R];
+    int row_head = hq;  // this lane's query head (SPLIT: R = 1)
 #pragma unroll
     for (int rb = 0; rb < R; ++rb) {
         qr[rb] = q0w + 16 * rb + (lane & 15);
+        if constexpr (SPLIT) {
+            row_head = hq + qr[rb] % group;
+            qr[rb] /= group;
+        }
         row_ok[rb] = qr[rb] < p.Nq;
-        q_off[rb] = ((int64_t)b * p.Nq + qr[rb]) * q_row_stride + (int64_t)hq * p.D;
+        q_off[rb] = ((int64_t)b * p.Nq + qr[rb]) * q_row_stride + (int64_t)row_head * p.D;
     }
 
     // Tangent presence: ALL instantiations have every tangent; the others
@@ -188,8 +240,15 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
 
     // Key range of the workgroup.
     int key_stop = p.Nk;
-    if (p.causal) key_stop = min(p.Nk, max(0, qtile * kBQ + kBQ + diag));
-    const int ntiles = (key_stop + kBK - 1) / kBK;
+    const int q_first = SPLIT ? q0w / group : q0w;  // query of the wavefront's first row
+    if (p.causal) key_stop = min(p.Nk, max(0, (SPLIT ? (qtile * kBQ + kBQ - 1) / group + 1 : qtile * kBQ + kBQ) + diag));
+    int ntiles = (key_stop + kBK - 1) / kBK;
+    int tile0 = 0;
+    if constexpr (SPLIT) {
+        const int per = (ntiles + p.splits - 1) / p.splits;
+        tile0 = min(ntiles, split * per);
+        ntiles = min(ntiles, tile0 + per);
+    }
     int klim[R];
 #pragma unroll
     for (int rb = 0; rb < R; ++rb) klim[rb] = p.causal ? min(p.Nk - 1, qr[rb] + diag) : p.Nk - 1;
@@ -224,7 +283,7 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
     const T* const tkbase = use_tk ? static_cast<const T*>(p.tk) + kv_base : nullptr;
     const T* const tvbase = use_tv ? static_cast<const T*>(p.tv) + kv_base : nullptr;
     auto tile_masked = [&](int k0) {
-        return (k0 + kBK > p.Nk) || (p.causal && k0 + kBK - 1 > q0w + diag);
+        return (k0 + kBK > p.Nk) || (p.causal && k0 + kBK - 1 > q_first + diag);
     };
     // A tile's keys are consumed in halves of 32 (key blocks 2h, 2h+1).
     auto apply_mask = [&](f32x4 (&s)[2], int k0, int h, int lim) {
@@ -487,6 +546,13 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
         wait_vmem();
         __syncthreads();  // tile t resident; every wavefront is done with tile t-1
         if (t + 1 < ntiles) issue_side(t + 1, nbuf, std::false_type{});
+        if constexpr (SPLIT) {
+            // Wavefronts past the last row only copy tiles.
+            if (q_first >= p.Nq) {
+                if (t + 1 < ntiles) issue_side(t + 1, nbuf, std::true_type{});
+                return;
+            }
+        }
 #pragma unroll
         for (int h = 0; h < FaTile<DP>::HALVES; ++h) {
             f32x4 s[R][2], ts[R][2];
@@ -520,11 +586,11 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
             if constexpr (JVP) __builtin_amdgcn_s_setprio(0);
         }
     };
-    if (ntiles > 0) {
-        issue_side(0, std::integral_constant<int, 0>{}, std::false_type{});
-        issue_side(0, std::integral_constant<int, 0>{}, std::true_type{});
+    if (ntiles > tile0) {
+        issue_side(tile0, std::integral_constant<int, 0>{}, std::false_type{});
+        issue_side(tile0, std::integral_constant<int, 0>{}, std::true_type{});
     }
-    for (int t = 0; t < ntiles; t += 2) {
+    for (int t = tile0; t < ntiles; t += 2) {
         step(t, std::integral_constant<int, 0>{});
         if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
     }
@@ -597,6 +663,26 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
         return;
     }
 
+    if constexpr (SPLIT) {
+        if (p.splits > 1) {
+            // The range's state; fa_combine_kernel joins the ranges.
+            const int64_t row = split * ((int64_t)p.B * p.Hq * p.Nq) + ((int64_t)b * p.Hq + row_head) * p.Nq + qr[0];
+            const f32x4 st = {m_run[0], row_sum4(l_lse[0]), row_sum4(l_run[0]), row_sum4(r_run[0])};
+            if (row_ok[0]) {
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    const int d = 16 * db + 4 * grp;
+                    if (d < p.D) {
+                        *reinterpret_cast<f32x4*>(p.ws_u + row * p.D + d) = u[0][db];
+                        if constexpr (JVP) *reinterpret_cast<f32x4*>(p.ws_g + row * p.D + d) = g[0][db];
+                    }
+                }
+                if (grp == 0) reinterpret_cast<f32x4*>(p.ws_st)[row] = st;
+            }
+            return;
+        }
+    }
+
     // ---- epilogue: O = U/l, tO = G/l - (r/l) O, LSE = m + log l ----
 #pragma unroll
     for (int rb = 0; rb < R; ++rb) {
@@ -624,7 +710,7 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
             }
         }
         if (MODE != FA_JVP && grp == 0 && row_ok[rb]) {
-            p.lse[((int64_t)b * p.Hq + hq) * p.Nq + qr[rb]] =
+            p.lse[((int64_t)b * p.Hq + row_head) * p.Nq + qr[rb]] =
                 empty ? __builtin_inff() : (m_run[rb] + log2f(l_lse_tot)) * kLn2;
         }
     }
@@ -676,6 +762,177 @@ void fa_fixup_kernel(const FaParams p) {
     fa_scan<T, DP, MODE, ALL, true>(p, kside0, kside1, vside0, vside1);
 }
 
+// FWD and FWD_JVP for grids that would leave CUs idle: workgroups of one row
+// block per wavefront (in the forward half of fa_kernel's rows), the heads of a
+// KV group packed into one tile when that takes fewer tiles (decoding: K and V
+// are then read once per KV head), and the keys of a tile split over p.splits
+// workgroups.  The rescaling scan never overflows, so no fixup launch follows;
+// with one split the workgroup writes its results itself.  Both modes take the
+// same key ranges, so their LSE is the same sum.
+template <typename T, int DP, int MODE, bool ALL>
+__global__ __launch_bounds__(FaTile<DP>::THREADS)
+__attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
+void fa_split_kernel(const FaParams p) {
+    FA_LDS_BUFFERS(T, DP, MODE);
+    fa_scan<T, DP, MODE, ALL, true, true>(p, kside0, kside1, vside0, vside1);
+}
+
+// The results of each row from its key ranges' states (one wavefront per row),
+// added in range order with weights w_s = 2^(m_s - m): O = sum w U / l,
+// tO = sum w G / l - (sum w r / l) O, LSE = m + log2(sum w lse_s).
+constexpr int kCombineRows = 4;
+template <typename T, int MODE>
+__global__ __launch_bounds__(64 * kCombineRows) void fa_combine_kernel(const FaParams p) {
+    constexpr bool JVP = MODE == FA_FWD_JVP;
+    const int lane = threadIdx.x & 63;
+    const int64_t rows = (int64_t)p.B * p.Hq * p.Nq;
+    const int64_t row = (int64_t)blockIdx.x * kCombineRows + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    // Lane s holds range s (at most 64); every lane ends with the totals.
+    const f32x4 mine = lane < p.splits ? reinterpret_cast<const f32x4*>(p.ws_st)[lane * rows + row]
+                                       : f32x4{-__builtin_inff(), 0.f, 0.f, 0.f};
+    const float m = wave_max(mine[0]);
+    const float w = mine[0] == -__builtin_inff() ? 0.f : fast_exp2(mine[0] - m);
+    const float l_lse = wave_sum(w * mine[1]);
+    const float l = JVP ? wave_sum(w * mine[2]) : l_lse;
+    const float r = JVP ? wave_sum(w * mine[3]) : 0.f;
+    const bool empty = !(l > 0.f);
+    const int d = 4 * lane < p.D ? 4 * lane : 0;
+    f32x4 au = {0.f, 0.f, 0.f, 0.f}, ag = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < p.splits; s0 += 4) {
+        f32x4 vu[4], vg[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t at = (min(s0 + i, p.splits - 1) * rows + row) * p.D + d;
+            vu[i] = *reinterpret_cast<const f32x4*>(p.ws_u + at);
+            if constexpr (JVP) vg[i] = *reinterpret_cast<const f32x4*>(p.ws_g + at);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // Lanes past the last range hold w = 0 (as does a range with no
+            // valid key, whose state is zero).
+            const float ws = __shfl(w, min(s0 + i, 63), 64);
+            if (s0 + i < p.splits) {
+                au += vu[i] * ws;
+                if constexpr (JVP) ag += vg[i] * ws;
+            }
+        }
+    }
+    const float inv = empty ? 0.f : 1.f / l;
+    const float rl = r * inv;
+    const int64_t bh = row / p.Nq;
+    if (4 * lane < p.D) {
+        const int64_t off = (((bh / p.Hq) * p.Nq + row % p.Nq) * p.Hq + bh % p.Hq) * p.D + d;
+        typename V<T>::x4 ov, tv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float o = au[e] * inv;
+            ov[e] = (T)o;
+            tv[e] = (T)(ag[e] * inv - rl * o);
+        }
+        *reinterpret_cast<typename V<T>::x4*>(static_cast<T*>(p.o) + off) = ov;
+        if constexpr (JVP) *reinterpret_cast<typename V<T>::x4*>(static_cast<T*>(p.to) + off) = tv;
+    }
+    if (lane == 0) p.lse[row] = empty ? __builtin_inff() : (m + log2f(l_lse)) * kLn2;
+}
+
+// How the forward modes cover a shape: splits = 0 is fa_kernel, otherwise
+// fa_split_kernel with that many key ranges per tile.
+struct FaSplitPlan {
+    int splits, pack, n_qtiles;
+};
+constexpr int kMaxSplits = 64;  // one lane of fa_combine_kernel each
+
+// The estimated time in units of one key tile of a full-size workgroup (1.2 us
+// at D = 64, 1.6 at 128 on MI355X): rounds of workgroups over the CUs times the
+// key tiles each scans.  Causal tiles differ in length: the longest one, or 1.5
+// times the mean load of a CU (resident workgroups pair long tiles with middle
+// ones), whichever is more.  A half-size workgroup's tile costs 0.8 of a full
+// one's (D > 128, where both have the same rows and rescaling spills: 1.35),
+// the fixup launch 3 tiles, the join of key ranges 5 and its traffic, written
+// once and read once, 7.8 MB a tile.  Measured, bf16, forward, us, fa_kernel
+// against the plan's choice:
+//   B=2, Nq=4, Nk=8192, H=32/8, D=128, causal     194 -> 18.5 (16 ranges, packed)
+//   B=1, Nq=1, Nk=20000, H=8/1, D=128             461 -> 19.0 (64 ranges, packed)
+//   B=1, N=333, H=16, D=64                        15.1 -> 10.1 (1 range)
+//   B=2, N=2048, H=8, D=128                       59.8 -> 46.8 (1 range)
+//   B=1, N=2500, H=16/4, D=128, causal            71.3 -> 52.8 (1 range)
+// and where it keeps fa_kernel: B=4, N=1024, H=16, D=128 42.7 against 53.1
+// (1 range); B=2, N=2500, H=16/4, causal 78.0 against 81.9.
+FaSplitPlan fa_split_plan(const FaParams& p, int cus) {
+    const int bq = p.D > 128 ? FaTile<256>::BQ : FaTile<128>::BQ;
+    const int bk = p.D > 128 ? FaTile<256>::BK : FaTile<128>::BK;
+    const int full_rows = p.D > 128 ? fa_rows<256, FA_FWD>() : fa_rows<128, FA_FWD>();
+    auto tiles = [](int64_t n, int64_t per) { return (n + per - 1) / per; };
+    const int64_t flat = (int64_t)p.B * p.Hq * tiles(p.Nq, bq);
+    const int64_t packed = (int64_t)p.B * p.Hkv * tiles((int64_t)p.group * p.Nq, bq);
+    FaSplitPlan plan{0, packed < flat ? 1 : 0, 0};
+    const int64_t base = plan.pack ? packed : flat;
+    plan.n_qtiles = (int)tiles(plan.pack ? (int64_t)p.group * p.Nq : p.Nq, bq);
+    const int64_t ntiles = tiles(p.Nk, bk);
+    const double seen = p.causal ? 1.0 - 0.5 * (p.Nq < p.Nk ? p.Nq : p.Nk) / p.Nk : 1.0;
+    auto cost = [&](int64_t blocks, int64_t longest) {
+        if (!p.causal) return (double)(tiles(blocks, cus) * longest);
+        const double load = 1.5 * blocks * (seen * longest) / cus;
+        return load > longest ? load : (double)longest;
+    };
+    double best = cost((int64_t)p.B * p.Hq * tiles(p.Nq, full_rows), ntiles) + 3.0;
+    const double half = p.D > 128 ? 1.35 : 0.8;
+    const double traffic = (double)p.B * p.Hq * p.Nq * p.D * 8.0 / 7.8e6;
+    for (int s = 1; s <= kMaxSplits && (s == 1 || 2 * s <= ntiles) && (s == 1 || base * s <= 4 * (int64_t)cus); ++s) {
+        const double c = half * cost(base * s, tiles(ntiles, s)) + (s > 1 ? 5.0 + s * traffic : 0.0);
+        if (c < 0.95 * best) {  // clearly better than the plan with fewer workgroups
+            best = c;
+            plan.splits = s;
+        }
+    }
+    return plan;
+}
+
+int64_t fa_split_ws_bytes(const FaParams& p, const FaSplitPlan& plan, int mode) {
+    if (plan.splits <= 1) return 0;
+    return (int64_t)plan.splits * p.B * p.Hq * p.Nq * ((mode == FA_FWD_JVP ? 2 : 1) * p.D + 4) * (int64_t)sizeof(float);
+}
+
+template <typename T, int MODE, bool ALL>
+int launch_split(FaParams p, const FaSplitPlan& plan, int dp, void* ws, hipStream_t stream) {
+    p.splits = plan.splits;
+    p.pack = plan.pack;
+    p.n_qtiles = plan.n_qtiles;
+    const int64_t rows = (int64_t)p.B * p.Hq * p.Nq;
+    p.ws_st = static_cast<float*>(ws);
+    p.ws_u = p.ws_st + (int64_t)p.splits * rows * 4;
+    p.ws_g = p.ws_u + (int64_t)p.splits * rows * p.D;
+    const int64_t blocks = (int64_t)p.n_qtiles * (p.pack ? p.Hkv : p.Hq) * p.B * p.splits;
+    if (blocks > 0x7fffffff) {
+        set_error("fa: grid too large");
+        return KF_E_UNSUPPORTED;
+    }
+    auto launch = [&](auto dpc) {
+        constexpr int DP = decltype(dpc)::value;
+        hipLaunchKernelGGL((fa_split_kernel<T, DP, MODE, ALL>), dim3((unsigned)blocks), dim3(FaTile<DP>::THREADS), 0,
+                           stream, p);
+    };
+    switch (dp) {
+        case 32: launch(std::integral_constant<int, 32>{}); break;
+        case 64: launch(std::integral_constant<int, 64>{}); break;
+        case 128: launch(std::integral_constant<int, 128>{}); break;
+        default: launch(std::integral_constant<int, 256>{}); break;
+    }
+    if (int rc = check_launch("fa_split_kernel launch")) return rc;
+    if (p.splits == 1) return KF_OK;
+    hipLaunchKernelGGL((fa_combine_kernel<T, MODE>), dim3((unsigned)((rows + kCombineRows - 1) / kCombineRows)),
+                       dim3(64 * kCombineRows), 0, stream, p);
+    return check_launch("fa_combine_kernel launch");
+}
+
+template <typename T>
+int launch_split_mode(int mode, const FaParams& p, const FaSplitPlan& plan, int dp, void* ws, hipStream_t stream) {
+    if (mode == FA_FWD) return launch_split<T, FA_FWD, true>(p, plan, dp, ws, stream);
+    if (p.tq && p.tk && p.tv) return launch_split<T, FA_FWD_JVP, true>(p, plan, dp, ws, stream);
+    return launch_split<T, FA_FWD_JVP, false>(p, plan, dp, ws, stream);
+}
+
 template <typename T, int MODE, bool ALL>
 int launch_variant(const FaParams& p, int dp, hipStream_t stream) {
     const int64_t blocks = (int64_t)p.n_qtiles * p.Hq * p.B;
@@ -709,7 +966,11 @@ int launch_mode(const FaParams& p, int dp, hipStream_t stream) {
     return launch_variant<T, MODE, false>(p, dp, stream);
 }
 
-int fa_dispatch(int mode, FaParams p, int dtype, hipStream_t stream) {
+// ws / ws_bytes: the split forward's workspace (FWD, FWD_JVP); a call that was
+// given none where its plan needs one runs fa_kernel.  forced: a plan's splits
+// and pack instead of the shape's own (n_qtiles is filled in).
+int fa_dispatch(int mode, FaParams p, int dtype, hipStream_t stream, void* ws = nullptr, int64_t ws_bytes = 0,
+                const FaSplitPlan* forced = nullptr) {
     KF_REQUIRE(p.B >= 0 && p.Nq >= 0 && p.Nk >= 0 && p.Hq > 0 && p.Hkv > 0, KF_E_INVALID,
                "fa: bad shape");
     KF_REQUIRE(p.Hq % p.Hkv == 0, KF_E_INVALID, "fa: Hq %% Hkv != 0");
@@ -729,6 +990,22 @@ int fa_dispatch(int mode, FaParams p, int dtype, hipStream_t stream) {
     if (mode != FA_FWD && p.Nk == 0) {
         // No keys: O = 0 and tO = 0 by the empty-row convention; the kernel
         // handles it with zero tiles.
+    }
+    if (mode != FA_JVP && p.Nk > 0) {
+        FaSplitPlan plan = forced ? *forced : fa_split_plan(p, device_cu_count());
+        if (forced) {
+            const int64_t rows = plan.pack ? (int64_t)p.group * p.Nq : p.Nq;
+            const int tile = dp > 128 ? FaTile<256>::BQ : FaTile<128>::BQ;
+            plan.n_qtiles = (int)((rows + tile - 1) / tile);
+        }
+        // One range: the fused mode's rescaling scan gains nothing over
+        // fa_kernel, which has the same 128 rows (92 against 88 us at B=2,
+        // N=2048, H=8, D=128; 15.2 against 16.3 at B=1, N=333, H=16, D=64).
+        if (!forced && mode == FA_FWD_JVP && plan.splits == 1) plan.splits = 0;
+        const int64_t need = fa_split_ws_bytes(p, plan, mode);
+        if (plan.splits > 0 && (need == 0 || (ws && ws_bytes >= need)))
+            return dtype == KF_BF16 ? launch_split_mode<bf16>(mode, p, plan, dp, ws, stream)
+                                    : launch_split_mode<f16>(mode, p, plan, dp, ws, stream);
     }
     if (dtype == KF_BF16) {
         switch (mode) {
@@ -772,6 +1049,71 @@ extern "C" int kf_fa_fwd(const void* q, const void* k, const void* v, void* o, f
     return fa_dispatch(FA_FWD, make_params(q, k, v, nullptr, nullptr, nullptr, o, lse, nullptr, B,
                                            Nq, Nk, Hq, Hkv, D, scale, causal),
                        dtype, static_cast<hipStream_t>(stream));
+}
+
+namespace kf {
+namespace {
+int64_t fwd_workspace_bytes(int mode, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                            int causal) {
+    if (!dims_fit(B, Nq, Nk, Hq, Hkv, D) || Hq <= 0 || Hkv <= 0 || Hq % Hkv || D <= 0 || D > 256) return -1;
+    if (B == 0 || Nq == 0 || Nk == 0) return 0;
+    FaParams p = make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, Nq,
+                             Nk, Hq, Hkv, D, 1.f, causal);
+    p.group = p.Hq / p.Hkv;
+    return fa_split_ws_bytes(p, fa_split_plan(p, device_cu_count()), mode);
+}
+}  // namespace
+}  // namespace kf
+
+extern "C" int64_t kf_fa_fwd_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                                             int causal) {
+    return kf::fwd_workspace_bytes(kf::FA_FWD, B, Nq, Nk, Hq, Hkv, D, causal);
+}
+
+extern "C" int64_t kf_fa_fwd_jvp_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
+                                                 int64_t D, int causal) {
+    return kf::fwd_workspace_bytes(kf::FA_FWD_JVP, B, Nq, Nk, Hq, Hkv, D, causal);
+}
+
+extern "C" int kf_fa_fwd_jvp_ws(const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                                const void* tv, void* o, float* lse, void* to, void* workspace,
+                                int64_t workspace_bytes, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
+                                int64_t D, float scale, int causal, int dtype, kf_stream_t stream) {
+    using namespace kf;
+    KF_REQUIRE(dims_fit(B, Nq, Nk, Hq, Hkv, D), KF_E_INVALID, "fa: shape out of range");
+    KF_REQUIRE((uintptr_t)workspace % 16 == 0, KF_E_WORKSPACE, "fa: workspace must be 16-byte aligned");
+    return fa_dispatch(FA_FWD_JVP, make_params(q, k, v, tq, tk, tv, o, lse, to, B, Nq, Nk, Hq, Hkv, D, scale, causal),
+                       dtype, static_cast<hipStream_t>(stream), workspace, workspace_bytes);
+}
+
+extern "C" int kf_fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
+                            int64_t workspace_bytes, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
+                            int64_t D, float scale, int causal, int dtype, kf_stream_t stream) {
+    using namespace kf;
+    KF_REQUIRE(dims_fit(B, Nq, Nk, Hq, Hkv, D), KF_E_INVALID, "fa: shape out of range");
+    KF_REQUIRE((uintptr_t)workspace % 16 == 0, KF_E_WORKSPACE, "fa: workspace must be 16-byte aligned");
+    return fa_dispatch(FA_FWD, make_params(q, k, v, nullptr, nullptr, nullptr, o, lse, nullptr, B,
+                                           Nq, Nk, Hq, Hkv, D, scale, causal),
+                       dtype, static_cast<hipStream_t>(stream), workspace, workspace_bytes);
+}
+
+// Test entry point (not in the public header): kf_fa_fwd_ws, or kf_fa_fwd_jvp_ws
+// when `to` is not null, with the split kernels forced to `splits` key ranges
+// (0: fa_kernel) with packed rows or not.
+extern "C" int kfm_fa_fwd_split(const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                                const void* tv, void* o, float* lse, void* to, void* workspace,
+                                int64_t workspace_bytes, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
+                                int64_t D, float scale, int causal, int dtype, int splits, int pack,
+                                kf_stream_t stream) {
+    using namespace kf;
+    KF_REQUIRE(dims_fit(B, Nq, Nk, Hq, Hkv, D) && Hkv > 0, KF_E_INVALID, "fa: shape out of range");
+    KF_REQUIRE(splits >= 0 && splits <= kMaxSplits, KF_E_INVALID, "fa: splits must be 0..%d", kMaxSplits);
+    const int mode = to ? FA_FWD_JVP : FA_FWD;
+    const FaParams p = make_params(q, k, v, tq, tk, tv, o, lse, to, B, Nq, Nk, Hq, Hkv, D, scale, causal);
+    const FaSplitPlan forced{splits, pack ? 1 : 0, 0};
+    KF_REQUIRE(workspace_bytes >= fa_split_ws_bytes(p, forced, mode) && (splits <= 1 || workspace), KF_E_WORKSPACE,
+               "fa: split workspace too small");
+    return fa_dispatch(mode, p, dtype, static_cast<hipStream_t>(stream), workspace, workspace_bytes, &forced);
 }
 
 extern "C" int kf_fa_jvp(const void* q, const void* k, const void* v, const void* tq,

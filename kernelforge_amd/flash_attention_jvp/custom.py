@@ -101,6 +101,13 @@ def _check_cached(q, out, lse):
         raise ValueError("lse must be float32 [B, Hq, Nq] on q's device")
 
 
+def _split_workspace(nbytes: int, device: torch.device) -> tuple[torch.Tensor | None, int]:
+    """The workspace a small grid's split kernels take (None when the shape takes none)."""
+    if nbytes <= 0:
+        return None, 0
+    return torch.empty(nbytes, device=device, dtype=torch.uint8), nbytes
+
+
 # ---------------------------------------------------------------------------
 # Opaque operators (C ABI launches on the current stream).
 # ---------------------------------------------------------------------------
@@ -110,10 +117,12 @@ def _fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
     B, Nq, Nk, Hq, Hkv, D = _dims(q, k)
     out = torch.empty_like(q)
     lse = torch.empty((B, Hq, Nq), device=q.device, dtype=torch.float32)
-    rc = _lib.load().kf_fa_fwd(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse),
-                               B, Nq, Nk, Hq, Hkv, D, scale, int(causal), _lib.kf_dtype(q.dtype),
-                               _lib.stream_of(q))
-    _lib.check(rc, "kf_fa_fwd")
+    lib = _lib.load()
+    ws, ws_bytes = _split_workspace(lib.kf_fa_fwd_workspace_bytes(B, Nq, Nk, Hq, Hkv, D, int(causal)), q.device)
+    rc = lib.kf_fa_fwd_ws(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws),
+                          ws_bytes, B, Nq, Nk, Hq, Hkv, D, scale, int(causal), _lib.kf_dtype(q.dtype),
+                          _lib.stream_of(q))
+    _lib.check(rc, "kf_fa_fwd_ws")
     return out, lse
 
 
@@ -162,11 +171,12 @@ def _fwd_jvp_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tq: torch.Ten
     out = torch.empty_like(q)
     tout = torch.empty_like(q)
     lse = torch.empty((B, Hq, Nq), device=q.device, dtype=torch.float32)
-    rc = _lib.load().kf_fa_fwd_jvp(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(tq), _lib.ptr(tk),
-                                   _lib.ptr(tv), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(tout),
-                                   B, Nq, Nk, Hq, Hkv, D, scale, int(causal), _lib.kf_dtype(q.dtype),
-                                   _lib.stream_of(q))
-    _lib.check(rc, "kf_fa_fwd_jvp")
+    lib = _lib.load()
+    ws, ws_bytes = _split_workspace(lib.kf_fa_fwd_jvp_workspace_bytes(B, Nq, Nk, Hq, Hkv, D, int(causal)), q.device)
+    rc = lib.kf_fa_fwd_jvp_ws(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(tq), _lib.ptr(tk), _lib.ptr(tv),
+                              _lib.ptr(out), _lib.ptr(lse), _lib.ptr(tout), _lib.ptr(ws), ws_bytes,
+                              B, Nq, Nk, Hq, Hkv, D, scale, int(causal), _lib.kf_dtype(q.dtype), _lib.stream_of(q))
+    _lib.check(rc, "kf_fa_fwd_jvp_ws")
     return out, lse, tout
 
 
