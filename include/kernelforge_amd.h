@@ -418,6 +418,14 @@ int kf_fa_fwd_jvp_ws(const void* q, const void* k, const void* v, const void* tq
 int64_t kf_fa_bwd_workspace_bytes(int64_t B, int64_t Nq, int64_t Hq, int64_t D);
 
 /*
+ * kf_fa_bwd with a workspace of this size (at least kf_fa_bwd_workspace_bytes,
+ * 16-byte aligned) may split a key tile's query rows over several workgroups
+ * where its grid would leave CUs idle; with less it runs unsplit.
+ */
+int64_t kf_fa_bwd_split_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                                        int causal);
+
+/*
  * Gradients dq, dk, dv (layouts of q, k, v) of the attention output for the
  * output cotangent dout [B, Nq, Hq, D], from the forward's o and natural-log
  * lse (P = exp(scale*q k^T - lse), recomputed; +inf rows contribute 0):

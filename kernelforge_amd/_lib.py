@@ -96,6 +96,7 @@ SIGNATURES = {
          _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
     ),
     "kf_fa_bwd_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
+    "kf_fa_bwd_split_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
     "kf_fa_bwd": (
         _int,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
@@ -131,6 +132,12 @@ MEASURE_SIGNATURES = {
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
          _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64,
          _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _int, _c_void_p],
+    ),
+    "kfm_fa_bwd_split": (
+        _int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64,
+         _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _int, _int, _c_void_p],
     ),
 }
 

@@ -10,7 +10,7 @@
 // P is recomputed from the forward's natural-log LSE; rows with LSE = +inf
 // (no valid key) get P = 0 and contribute nothing.
 //
-// Two launches, no atomics, deterministic:
+// Two launches (three where key tiles are split), no atomics, deterministic:
 //   1. dq kernel, one workgroup per (query tile, batch, query head), shaped
 //      like the forward: lane l owns query row l%16 and computes S^T = K Q^T
 //      and dP^T = V dO^T over K/V tiles streamed through LDS, then
@@ -21,7 +21,9 @@
 //      (plus their LSE/Delta entries) of every query head of the group, in a
 //      fixed order, computes S = Q K^T and dP = dO V^T with the key as the
 //      output column, and accumulates dV^T += dO^T P and dK^T += Q^T dS with
-//      dO^T and Q^T read by transposing LDS reads.  Up to D = 128 on grids
+//      dO^T and Q^T read by transposing LDS reads.  On grids that leave CUs
+//      idle several workgroups share a key tile's query tiles and a third
+//      launch adds their fp32 partial sums in order.  Up to D = 128 on grids
 //      that fill the chip (causal: D = 64 and 128), each wavefront owns two
 //      key blocks (four at D = 32; K in registers, V in LDS), so each
 //      transposed operand feeds four (eight) MFMAs; otherwise one block,
@@ -47,12 +49,15 @@ struct FaBwdParams {
     float* ws_lse2;   // [B][Hq][nq_pad]: LSE * log2(e), +inf for rows >= Nq
     float* ws_delta;  // [B][Hq][nq_pad]: Delta, 0 for rows >= Nq
     int B, Nq, Nk, Hq, Hkv, D, group;
-    int n_qtiles;  // query tiles of dq_rows() rows (dq grid)
+    int n_qtiles;  // query tiles (dq grid)
     int n_ktiles;  // key tiles of FaTile::BQ keys (one-block dkdv grid)
     int nq_pad;    // query rows padded to a multiple of FaTile::BQ
     float scale;
     float scale_log2;
     int causal;
+    int ksplits;      // dK/dV workgroups per key tile (each takes a run of its query tiles)
+    float* ws_dk;     // [ksplits][B][Nk][Hkv][D] partial sums of dK / scale and dV (ksplits > 1)
+    float* ws_dv;
 };
 
 // XCD-aware renumbering: the hardware sends block i to XCD i % 8; give each
@@ -77,15 +82,14 @@ __device__ __forceinline__ typename V<T>::x8 load_row8(const T* p, bool ok) {
 // Row blocks of 16 query rows per wavefront: two up to D = 128 (a 256-row
 // workgroup), so that every K row and K^T / V operand read from LDS feeds two
 // MFMAs and each tile copy serves twice the rows; one at D = 256.
+// Grids that would leave CUs idle take one block up to D = 128 too.
 template <int DP> constexpr int dq_row_blocks() { return DP <= 128 ? 2 : 1; }
-template <int DP> constexpr int dq_rows() { return FaTile<DP>::BQ * dq_row_blocks<DP>(); }
 
-template <typename T, int DP>
+template <typename T, int DP, int R>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
 void fa_bwd_dq_kernel(const FaBwdParams p) {
-    constexpr int R = dq_row_blocks<DP>();
-    constexpr int kBQ = dq_rows<DP>(), kBK = FaTile<DP>::BK;
+    constexpr int kBQ = FaTile<DP>::BQ * R, kBK = FaTile<DP>::BK;
     constexpr int DS = DP / 32, DB = DP / 16;
     typedef typename V<T>::x8 x8;
     // Double-buffered K and V tiles, one LDS variable per buffer so that the
@@ -364,9 +368,13 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = lane >> 4;
 
-    const int logical = xcd_logical_block();
+    // Causal runs of a split key tile differ in length: longest first.
+    const int xlogical = xcd_logical_block();
+    const int logical = p.causal && p.ksplits > 1 ? causal_tile_order(xlogical, p.n_ktiles) : xlogical;
     const int ktile = logical % p.n_ktiles;
-    const int rest = logical / p.n_ktiles;
+    int rest = logical / p.n_ktiles;
+    const int split = rest % p.ksplits;
+    rest /= p.ksplits;
     const int hk = rest % p.Hkv, b = rest / p.Hkv;
 
     const int k0 = ktile * kBKEYS;             // first key of the workgroup
@@ -393,7 +401,10 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
     const int n_rt = (p.Nq + kBR - 1) / kBR;
     const int rt0 = p.causal ? min(n_rt, max(0, k0 - diag) / kBR) : 0;
     const int per_head = n_rt - rt0;
-    const int ntiles = per_head * p.group;
+    // This workgroup's run of the (head, row tile) sequence.
+    const int per_split = (per_head * p.group + p.ksplits - 1) / p.ksplits;
+    const int u0 = min(per_head * p.group, split * per_split);
+    const int ntiles = min(per_head * p.group, u0 + per_split);
     const float c = p.scale_log2;
 
     const uint32_t voff = full_tile_shortcut<DP>() ? full_tile_lane_offset<T, DP>(q_row_stride, wave, lane) : 0u;
@@ -530,10 +541,23 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
             __builtin_amdgcn_s_setprio(0);
         }
     };
-    if (ntiles > 0) issue(0, std::integral_constant<int, 0>{});
-    for (int u = 0; u < ntiles; u += 2) {
+    if (ntiles > u0) issue(u0, std::integral_constant<int, 0>{});
+    for (int u = u0; u < ntiles; u += 2) {
         step(u, std::integral_constant<int, 0>{});
         if (u + 1 < ntiles) step(u + 1, std::integral_constant<int, 1>{});
+    }
+
+    if (p.ksplits > 1) {
+        const int64_t part = split * ((int64_t)p.B * p.Nk * kv_row_stride) + kv_off;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            const int d = 16 * db + 4 * grp;
+            if (key_ok && d < p.D) {
+                *reinterpret_cast<f32x4*>(p.ws_dk + part + d) = dk[db];
+                *reinterpret_cast<f32x4*>(p.ws_dv + part + d) = dv[db];
+            }
+        }
+        return;
     }
 
     // dK = scale * dS^T Q, dV = P^T dO; lane holds key kr, d = 16*db + 4*grp + 0..3.
@@ -615,7 +639,9 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
     const int n_kt = (p.Nk + kBKEYS - 1) / kBKEYS;
     const int logical = p.causal ? causal_tile_order(xcd_logical_block(), n_kt) : xcd_logical_block();
     const int ktile = logical % n_kt;
-    const int rest = logical / n_kt;
+    int rest = logical / n_kt;
+    const int split = rest % p.ksplits;
+    rest /= p.ksplits;
     const int hk = rest % p.Hkv, b = rest / p.Hkv;
 
     const int k0 = ktile * kBKEYS;  // first key of the workgroup
@@ -649,7 +675,10 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
     const int n_rt = (p.Nq + kBR - 1) / kBR;
     const int rt0 = p.causal ? min(n_rt, max(0, k0 - diag) / kBR) : 0;
     const int per_head = n_rt - rt0;
-    const int ntiles = per_head * p.group;
+    // This workgroup's run of the (head, row tile) sequence.
+    const int per_split = (per_head * p.group + p.ksplits - 1) / p.ksplits;
+    const int u0 = min(per_head * p.group, split * per_split);
+    const int ntiles = min(per_head * p.group, u0 + per_split);
     const float c = p.scale_log2;
 
     const uint32_t voff = panel_lane_offset<T>(q_row_stride, lane);
@@ -809,12 +838,12 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
             __builtin_amdgcn_s_setprio(0);
         }
     };
-    if (ntiles > 0) issue(0, std::integral_constant<int, 0>{});
-    for (int u = 0; u < ntiles; u += 2) {
+    if (ntiles > u0) issue(u0, std::integral_constant<int, 0>{});
+    for (int u = u0; u < ntiles; u += 2) {
         step(u, std::integral_constant<int, 0>{});
         if (u + 1 < ntiles) step(u + 1, std::integral_constant<int, 1>{});
     }
-    if (ntiles == 0) wait_vmem();  // the V copies land before the workgroup ends
+    if (ntiles == u0) wait_vmem();  // the V copies land before the workgroup ends
 
     // dK = scale * dS^T Q, dV = P^T dO; lane holds key k0w + 16*kb + l%16,
     // d = 16*db + 4*grp + 0..3.  The lane index passes through an empty asm
@@ -826,6 +855,18 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
     for (int kb = 0; kb < KB; ++kb) {
         const int kr = k0w + 16 * kb + (lane_out & 15);
         const int64_t kv_off = kv_base + (int64_t)kr * kv_row_stride;
+        if (p.ksplits > 1) {
+            const int64_t part = split * ((int64_t)p.B * p.Nk * kv_row_stride) + kv_off;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const int d = 16 * db + 4 * (lane_out >> 4);
+                if (kr < p.Nk && d < p.D) {
+                    *reinterpret_cast<f32x4*>(p.ws_dk + part + d) = dk[kb][db];
+                    *reinterpret_cast<f32x4*>(p.ws_dv + part + d) = dv[kb][db];
+                }
+            }
+            continue;
+        }
         T* const dkrow = static_cast<T*>(p.dk) + kv_off;
         T* const dvrow = static_cast<T*>(p.dv) + kv_off;
 #pragma unroll
@@ -853,59 +894,171 @@ int64_t padded_rows(int64_t Nq, int64_t D) {
     return D > 128 ? nq_pad_of<256>(Nq) : nq_pad_of<128>(Nq);
 }
 
-// key_blocks: 16-key blocks per wavefront of the dK/dV kernel, 0 = chosen per
-// shape; 1 or 2 force one kernel (kfm_fa_bwd_blocks, so tests reach both).
+// dK and dV from the splits' partial sums, in split order.
+template <typename T>
+__global__ __launch_bounds__(256) void fa_bwd_join_kernel(const FaBwdParams p, int64_t n4) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const f32x4* dk = reinterpret_cast<const f32x4*>(p.ws_dk) + i;
+    const f32x4* dv = reinterpret_cast<const f32x4*>(p.ws_dv) + i;
+    f32x4 ak = {0.f, 0.f, 0.f, 0.f}, av = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < p.ksplits; s0 += 2) {
+        const int s1 = min(s0 + 1, p.ksplits - 1);
+        const f32x4 k0 = dk[s0 * n4], v0 = dv[s0 * n4], k1 = dk[s1 * n4], v1 = dv[s1 * n4];
+        ak += k0;
+        av += v0;
+        if (s0 + 1 < p.ksplits) {
+            ak += k1;
+            av += v1;
+        }
+    }
+    typename V<T>::x4 rk, rv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        rk[e] = (T)(ak[e] * p.scale);
+        rv[e] = (T)av[e];
+    }
+    reinterpret_cast<typename V<T>::x4*>(p.dk)[i] = rk;
+    reinterpret_cast<typename V<T>::x4*>(p.dv)[i] = rv;
+}
+
+// How the backward covers a shape: the dK/dV kernel (several key blocks per
+// wavefront or one) with its workgroups per key tile, and the dQ kernel's row
+// blocks per wavefront.
+struct FaBwdPlan {
+    bool wide;
+    int ksplits, dq_blocks;
+};
+constexpr int kMaxKeySplits = 16;
+
+// Both kernels run one workgroup per CU.  Two key blocks per wavefront (half
+// the workgroups, each doing twice the work at fewer LDS reads per product)
+// once the grid gives every CU more than half a workgroup; under a causal
+// mask, with the longest key tiles started first (causal_tile_order), that is
+// faster at D = 128 and 64 (B=2, H=16, N=4096 on MI355X: 416 against 470 us
+// and 258 against 296 us for the whole backward) but not at D = 32, whose
+// 512-key workgroups and the wavefronts within one do too unequal work (245
+// against 229 us).
+//
+// From there the plan splits each key tile's query tiles over several
+// workgroups, or takes the other kernel, where the estimate improves by a
+// tenth.  The estimate counts query tiles of the one-block kernel: rounds of
+// workgroups times tiles (causal: the longest workgroup or the mean load of a
+// CU), a two-block workgroup's tile 1.62 and the four-block one's (D = 32) 2.5
+// of a one-block one's; splitting adds a launch and the partial sums' traffic.
+// Measured, whole backward, us, unsplit against the plan's choice:
+//   B=2, N=2500, H=16/4, D=128, causal     375 -> 226 (one block, 3 splits)
+//   B=1, N=1500, H=16/2, D=64, causal      263 -> 62
+//   B=1, Nq=4096, Nk=300, H=16, D=128      144 -> 68 (4)
+//   B=1, N=300, H=32/8, D=128               55 -> 38
+//   B=1, N=2000, H=8/4, D=256              291 -> 209 (2)
+// and unsplit where that is faster: B=2, N=2048, H=8, D=128 126 against 145.
+// A caller whose workspace holds no partial sums takes max_splits = 1.
+FaBwdPlan fa_bwd_plan(const FaBwdParams& p, int dp, int cus, int max_splits = kMaxKeySplits) {
+    auto tiles = [](int64_t n, int64_t per) { return (n + per - 1) / per; };
+    const int bq = dp > 128 ? FaTile<256>::BQ : FaTile<128>::BQ, bk = dp > 128 ? FaTile<256>::BK : FaTile<128>::BK;
+    const int wide_keys = dp <= 32 ? dkdv_wide_keys<32>() : dkdv_wide_keys<128>();
+    const int64_t heads = (int64_t)p.B * p.Hkv;
+    const int64_t n1 = heads * tiles(p.Nk, bq), nw = heads * tiles(p.Nk, wide_keys);
+    FaBwdPlan plan{false, 1, 1};
+    plan.wide = dp <= 128 && (!p.causal || dp > 32) && 2 * nw > cus;
+
+    const int64_t units = tiles(p.Nq, bk) * p.group;  // query tiles of one key tile
+    const double seen = p.causal ? 1.0 - 0.5 * (p.Nk < p.Nq ? p.Nk : p.Nq) / p.Nq : 1.0;
+    const double unit_us = dp <= 32 ? 0.7 : dp <= 64 ? 1.1 : 1.9;
+    const double join = 4.0 / unit_us, traffic = 16.0 * heads * p.Nk * p.D / (7e6 * unit_us);
+    auto cost = [&](bool wide, int s) {
+        const int64_t blocks = (wide ? nw : n1) * s, longest = tiles(units, s);
+        const double tile = !wide ? 1.0 : dp <= 32 ? 2.5 : 1.62;
+        double t = (double)(tiles(blocks, cus) * longest);
+        if (p.causal) {
+            const double load = 1.1 * blocks * seen * longest / cus;
+            t = load > longest ? load : (double)longest;
+        }
+        return t * tile + (s > 1 ? join + s * traffic : 0.0);
+    };
+    double best = cost(plan.wide, 1);
+    for (int w = 0; w <= (dp <= 128 ? 1 : 0); ++w)
+        for (int s = 1; s <= max_splits && (s == 1 || 2 * s <= units); ++s) {
+            const double c = cost(w != 0, s);
+            if (c < 0.9 * best) {
+                best = c;
+                plan.wide = w != 0;
+                plan.ksplits = s;
+            }
+        }
+
+    // dQ: two row blocks per wavefront unless half-size workgroups, whose key
+    // tile costs 0.8 of a full one's, come out clearly ahead.
+    if (dp <= 128) {
+        const int64_t full = (int64_t)p.B * p.Hq * tiles(p.Nq, 2 * bq), half = (int64_t)p.B * p.Hq * tiles(p.Nq, bq);
+        auto dq_cost = [&](int64_t blocks) {
+            const double load = blocks * seen / cus;
+            return p.causal ? (load > 1.0 ? load : 1.0) : (double)tiles(blocks, cus);
+        };
+        plan.dq_blocks = 0.8 * dq_cost(half) < 0.95 * dq_cost(full) ? 1 : 2;
+    }
+    return plan;
+}
+
+int64_t fa_bwd_partial_bytes(const FaBwdParams& p, int ksplits) {
+    return ksplits > 1 ? 2 * (int64_t)sizeof(float) * ksplits * p.B * p.Nk * p.Hkv * p.D : 0;
+}
+
 template <typename T, int DP>
-int launch_bwd(const FaBwdParams& p, int key_blocks, hipStream_t stream) {
+int launch_bwd(FaBwdParams p, const FaBwdPlan& plan, hipStream_t stream) {
+    const int dq_rows = FaTile<DP>::BQ * plan.dq_blocks;
+    p.n_qtiles = (p.Nq + dq_rows - 1) / dq_rows;
+    p.ksplits = plan.ksplits;
     const int64_t qblocks = (int64_t)p.n_qtiles * p.Hq * p.B;
-    int64_t kblocks = (int64_t)p.n_ktiles * p.Hkv * p.B;
-    // Two key blocks per wavefront (half the workgroups, each doing twice the
-    // work at fewer LDS reads per product) once the grid still gives every
-    // CU more than half a workgroup; both kernels run one workgroup per CU.
-    // Under a causal mask, with the longest key tiles started first
-    // (causal_tile_order), it is faster at D = 128 and 64 (B=2, H=16,
-    // N=4096 on MI355X: 416 against 470 us and 258 against 296 us for the
-    // whole backward) but not at D = 32, whose 512-key workgroups and the
-    // wavefronts within one do too unequal work (245 against 229 us).
-    bool wide = false;
+    int64_t kblocks = (int64_t)p.n_ktiles * p.Hkv * p.B * p.ksplits;
     if constexpr (DP <= 128) {
-        const int64_t wblocks = ((int64_t)p.Nk + dkdv_wide_keys<DP>() - 1) / dkdv_wide_keys<DP>() * p.Hkv * p.B;
-        wide = key_blocks ? key_blocks == 2
-                                     : (!p.causal || DP > 32) && 2 * wblocks > device_cu_count();
-        if (wide) kblocks = wblocks;
+        if (plan.wide)
+            kblocks = ((int64_t)p.Nk + dkdv_wide_keys<DP>() - 1) / dkdv_wide_keys<DP>() * p.Hkv * p.B * p.ksplits;
     }
     if (qblocks > 0x7fffffff || kblocks > 0x7fffffff) {
         set_error("fa_bwd: grid too large");
         return KF_E_UNSUPPORTED;
     }
+    const dim3 threads(FaTile<DP>::THREADS);
     if (qblocks > 0) {
-        hipLaunchKernelGGL((fa_bwd_dq_kernel<T, DP>), dim3((unsigned)qblocks), dim3(FaTile<DP>::THREADS), 0,
-                           stream, p);
-        const int rc = check_launch("fa_bwd_dq_kernel launch");
-        if (rc != KF_OK) return rc;
+        if (plan.dq_blocks == 1)
+            hipLaunchKernelGGL((fa_bwd_dq_kernel<T, DP, 1>), dim3((unsigned)qblocks), threads, 0, stream, p);
+        else
+            hipLaunchKernelGGL((fa_bwd_dq_kernel<T, DP, dq_row_blocks<DP>()>), dim3((unsigned)qblocks), threads, 0,
+                               stream, p);
+        if (int rc = check_launch("fa_bwd_dq_kernel launch")) return rc;
     }
-    if (kblocks > 0) {
-        if constexpr (DP <= 128) {
-            if (wide) {
-                hipLaunchKernelGGL((fa_bwd_dkdv_wide_kernel<T, DP>), dim3((unsigned)kblocks),
-                                   dim3(FaTile<DP>::THREADS), 0, stream, p);
-                return check_launch("fa_bwd_dkdv_wide_kernel launch");
-            }
+    if (kblocks == 0) return KF_OK;
+    bool launched = false;
+    if constexpr (DP <= 128) {
+        if (plan.wide) {
+            hipLaunchKernelGGL((fa_bwd_dkdv_wide_kernel<T, DP>), dim3((unsigned)kblocks), threads, 0, stream, p);
+            if (int rc = check_launch("fa_bwd_dkdv_wide_kernel launch")) return rc;
+            launched = true;
         }
-        hipLaunchKernelGGL((fa_bwd_dkdv_kernel<T, DP>), dim3((unsigned)kblocks), dim3(FaTile<DP>::THREADS), 0,
-                           stream, p);
-        return check_launch("fa_bwd_dkdv_kernel launch");
     }
-    return KF_OK;
+    if (!launched) {
+        hipLaunchKernelGGL((fa_bwd_dkdv_kernel<T, DP>), dim3((unsigned)kblocks), threads, 0, stream, p);
+        if (int rc = check_launch("fa_bwd_dkdv_kernel launch")) return rc;
+    }
+    if (p.ksplits == 1) return KF_OK;
+    const int64_t n4 = (int64_t)p.B * p.Nk * p.Hkv * p.D / 4;
+    if ((n4 + 255) / 256 > 0x7fffff) {
+        set_error("fa_bwd: grid too large");
+        return KF_E_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL((fa_bwd_join_kernel<T>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, p, n4);
+    return check_launch("fa_bwd_join_kernel launch");
 }
 
 template <typename T>
-int launch_bwd_dp(const FaBwdParams& p, int dp, int key_blocks, hipStream_t stream) {
+int launch_bwd_dp(const FaBwdParams& p, int dp, const FaBwdPlan& plan, hipStream_t stream) {
     switch (dp) {
-        case 32: return launch_bwd<T, 32>(p, key_blocks, stream);
-        case 64: return launch_bwd<T, 64>(p, key_blocks, stream);
-        case 128: return launch_bwd<T, 128>(p, key_blocks, stream);
-        case 256: return launch_bwd<T, 256>(p, key_blocks, stream);
+        case 32: return launch_bwd<T, 32>(p, plan, stream);
+        case 64: return launch_bwd<T, 64>(p, plan, stream);
+        case 128: return launch_bwd<T, 128>(p, plan, stream);
+        case 256: return launch_bwd<T, 256>(p, plan, stream);
         default: set_error("fa_bwd: head dim %d not supported by this build", p.D); return KF_E_UNSUPPORTED;
     }
 }
@@ -928,10 +1081,16 @@ extern "C" int64_t kf_fa_bwd_workspace_bytes(int64_t B, int64_t Nq, int64_t Hq, 
 namespace kf {
 namespace {
 
+int bwd_pad_dim(int64_t D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256; }
+
+// key_blocks: 16-key blocks per wavefront of the dK/dV kernel, 0 = the plan's
+// choice; 1 or 2 force one kernel; ksplits > 0 forces the workgroups per key
+// tile (kfm_fa_bwd_blocks, kfm_fa_bwd_split: tests reach every path).  A plan
+// whose partial sums do not fit the workspace runs unsplit.
 int fa_bwd_run(const void* q, const void* k, const void* v, const void* o, const float* lse, const void* dout,
                void* dq, void* dk, void* dv, void* workspace, int64_t workspace_bytes, int64_t B, int64_t Nq,
                int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D, float scale, int causal, int dtype, int key_blocks,
-               kf_stream_t stream) {
+               int ksplits, kf_stream_t stream) {
     KF_REQUIRE(bwd_dims_fit(B, Nq, Nk, Hq, Hkv, D), KF_E_INVALID, "fa_bwd: shape out of range");
     KF_REQUIRE(Hq > 0 && Hkv > 0 && Hq % Hkv == 0, KF_E_INVALID, "fa_bwd: Hq must be a positive multiple of Hkv");
     KF_REQUIRE(D > 0 && D % 8 == 0 && D <= 256, KF_E_INVALID,
@@ -952,17 +1111,29 @@ int fa_bwd_run(const void* q, const void* k, const void* v, const void* o, const
     p.ws_delta = static_cast<float*>(workspace) + B * Hq * nq_pad;
     p.B = (int)B; p.Nq = (int)Nq; p.Nk = (int)Nk; p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.D = (int)D;
     p.group = (int)(Hq / Hkv);
-    const int dp = D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
+    const int dp = bwd_pad_dim(D);
     const int bq = dp > 128 ? FaTile<256>::BQ : FaTile<128>::BQ;
-    const int bq_dq = dp > 128 ? dq_rows<256>() : dq_rows<128>();
-    p.n_qtiles = (int)((Nq + bq_dq - 1) / bq_dq);
     p.n_ktiles = (int)((Nk + bq - 1) / bq);
     p.nq_pad = (int)nq_pad;
     p.scale = scale;
     p.scale_log2 = scale * kLog2e;
     p.causal = causal ? 1 : 0;
+    FaBwdPlan plan{false, 1, 1};
+    if (Nq > 0 && Nk > 0) plan = fa_bwd_plan(p, dp, device_cu_count());
+    if (key_blocks || ksplits) {
+        if (key_blocks) plan.wide = dp <= 128 && key_blocks == 2;
+        plan.ksplits = ksplits ? ksplits : 1;
+    }
+    const int64_t stats = (need + 255) / 256 * 256;
+    if (plan.ksplits > 1 &&
+        ((uintptr_t)workspace % 16 || workspace_bytes < stats + fa_bwd_partial_bytes(p, plan.ksplits))) {
+        KF_REQUIRE(ksplits == 0, KF_E_WORKSPACE, "fa_bwd: split workspace too small");
+        plan = fa_bwd_plan(p, dp, device_cu_count(), 1);
+    }
+    p.ws_dk = reinterpret_cast<float*>(static_cast<char*>(workspace) + stats);
+    p.ws_dv = p.ws_dk + (int64_t)plan.ksplits * B * Nk * Hkv * D;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    return dtype == KF_BF16 ? launch_bwd_dp<bf16>(p, dp, key_blocks, s) : launch_bwd_dp<f16>(p, dp, key_blocks, s);
+    return dtype == KF_BF16 ? launch_bwd_dp<bf16>(p, dp, plan, s) : launch_bwd_dp<f16>(p, dp, plan, s);
 }
 
 }  // namespace
@@ -974,7 +1145,21 @@ extern "C" int kf_fa_bwd(const void* q, const void* k, const void* v, const void
                          int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D, float scale, int causal,
                          int dtype, kf_stream_t stream) {
     return kf::fa_bwd_run(q, k, v, o, lse, dout, dq, dk, dv, workspace, workspace_bytes, B, Nq, Nk, Hq, Hkv, D,
-                          scale, causal, dtype, 0, stream);
+                          scale, causal, dtype, 0, 0, stream);
+}
+
+extern "C" int64_t kf_fa_bwd_split_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
+                                                   int64_t D, int causal) {
+    using namespace kf;
+    const int64_t need = kf_fa_bwd_workspace_bytes(B, Nq, Hq, D);
+    if (need < 0 || !bwd_dims_fit(B, Nq, Nk, Hq, Hkv, D) || Hkv <= 0 || Hq % Hkv) return -1;
+    if (B == 0 || Nq == 0 || Nk == 0) return need;
+    FaBwdParams p{};
+    p.B = (int)B; p.Nq = (int)Nq; p.Nk = (int)Nk; p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.D = (int)D;
+    p.group = (int)(Hq / Hkv);
+    p.causal = causal ? 1 : 0;
+    const FaBwdPlan plan = fa_bwd_plan(p, bwd_pad_dim(D), device_cu_count());
+    return plan.ksplits > 1 ? (need + 255) / 256 * 256 + fa_bwd_partial_bytes(p, plan.ksplits) : need;
 }
 
 // Test entry point (not in the public header): kf_fa_bwd with the dK/dV
@@ -987,5 +1172,19 @@ extern "C" int kfm_fa_bwd_blocks(const void* q, const void* k, const void* v, co
                                  int dtype, int key_blocks, kf_stream_t stream) {
     KF_REQUIRE(key_blocks >= 0 && key_blocks <= 2, KF_E_INVALID, "fa_bwd: key_blocks must be 0, 1 or 2");
     return kf::fa_bwd_run(q, k, v, o, lse, dout, dq, dk, dv, workspace, workspace_bytes, B, Nq, Nk, Hq, Hkv, D,
-                          scale, causal, dtype, key_blocks, stream);
+                          scale, causal, dtype, key_blocks, 0, stream);
+}
+
+// The same with the number of workgroups per key tile forced as well (1..16);
+// the workspace holds kf_fa_bwd_workspace_bytes, rounded up to 256, plus
+// 8 * splits * B * Nk * Hkv * D bytes.
+extern "C" int kfm_fa_bwd_split(const void* q, const void* k, const void* v, const void* o,
+                                const float* lse, const void* dout, void* dq, void* dk, void* dv,
+                                void* workspace, int64_t workspace_bytes, int64_t B, int64_t Nq,
+                                int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D, float scale, int causal,
+                                int dtype, int key_blocks, int splits, kf_stream_t stream) {
+    KF_REQUIRE(key_blocks >= 1 && key_blocks <= 2 && splits >= 1 && splits <= kf::kMaxKeySplits, KF_E_INVALID,
+               "fa_bwd: key_blocks must be 1 or 2 and splits 1..%d", kf::kMaxKeySplits);
+    return kf::fa_bwd_run(q, k, v, o, lse, dout, dq, dk, dv, workspace, workspace_bytes, B, Nq, Nk, Hq, Hkv, D,
+                          scale, causal, dtype, key_blocks, splits, stream);
 }

@@ -192,7 +192,7 @@ def _bwd_op(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     B, Nq, Nk, Hq, Hkv, D = _dims(q, k)
     lib = _lib.load()
     dq, dk, dv = (torch.empty_like(x, memory_format=torch.contiguous_format) for x in (q, k, v))
-    ws_bytes = lib.kf_fa_bwd_workspace_bytes(B, Nq, Hq, D)
+    ws_bytes = lib.kf_fa_bwd_split_workspace_bytes(B, Nq, Nk, Hq, Hkv, D, int(causal))
     if ws_bytes < 0:
         raise ValueError("flash attention backward: unsupported shape")
     ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)
