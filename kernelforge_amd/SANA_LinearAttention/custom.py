@@ -54,14 +54,24 @@ _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """The zero-initialised workspace of the current stream on `device`, at
-    least `nbytes` long (its control words are zero between calls)."""
+    least `nbytes` long (its control words are zero between calls).
+
+    Under graph capture the zeroing is recorded with every call instead: the
+    fill of a fresh tensor would only run when the graph that happened to
+    allocate it is replayed, while later graphs captured on the same stream
+    share the tensor."""
     stream = torch.cuda.current_stream(device)
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
+    capturing = torch.cuda.is_current_stream_capturing()
     with _ws_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
-            ws = torch.zeros(max(nbytes, 1 << 20), device=device, dtype=torch.uint8)
+            make = torch.empty if capturing else torch.zeros
+            ws = make(max(nbytes, 1 << 20), device=device, dtype=torch.uint8)
             _workspaces[key] = ws
+    if capturing:
+        rc = _lib.load().kf_linattn_workspace_init(_lib.ptr(ws), ws.numel(), ctypes.c_void_p(stream.cuda_stream))
+        _lib.check(rc, "kf_linattn_workspace_init")
     return ws
 
 

@@ -343,12 +343,12 @@ GROUPED_HEADS, GROUPED_DIM = 36, 32
 class GroupedFull64QOutLiteLA(JointLiteLA):
     """The reference's shape-specialised LiteLA (SANA_LinearAttention/custom.py:812-861),
     with its constructor checks: exactly B=1, N=1024, C=1152, H=36, D=32, bf16,
-    ``qk_norm=False``, ``use_bias=False``, and no ``rotary_emb``.  Like the
-    reference, it always runs the fused projection kernels (the k/v projection
-    with ReLU and the state partials, then the q projection with the output;
-    kf_litela_fused_attn), followed by the bias-fused output projection."""
-
-    fused_projection = True
+    ``qk_norm=False``, ``use_bias=False``, and no ``rotary_emb``.  The reference
+    fuses the projections with the attention here; on MI355X the fused kernels'
+    256-token tiles give this shape 48 workgroups, and the projection GEMM with
+    its small tiles followed by the attention kernel is faster (the block's
+    kernels 77 against 40 us), so the module leaves the choice to the shape rule
+    (``fused_projection = True`` still forces the fused kernels)."""
 
     def __init__(self, *args, **kwargs):
         batch, seq_len, dtype = kwargs.get("batch"), kwargs.get("seq_len"), kwargs.get("dtype")

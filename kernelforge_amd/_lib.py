@@ -121,6 +121,9 @@ MEASURE_SIGNATURES = {
         [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _i64,
          _c_void_p],
     ),
+    "kfm_proj_gemm_tile": (
+        _int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64, _i64, _int, _int, _int,
+               _c_void_p]),
     "kfm_linattn_split_plan": (_int, [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
     "kfm_fa_fwd_split": (
         _int,

@@ -47,7 +47,7 @@ template <typename T, typename C> struct StagedOut {
 };
 
 template <typename T, typename C, bool BIAS>
-__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2, C::MB * C::NB <= 8 ? 4 : 2)))
 void proj_gemm_kernel(GemmParams p) {
     __shared__ __attribute__((aligned(16))) T lds[C::STAGES * (C::XS + C::WS)];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -137,6 +137,13 @@ template <typename T, int BN, bool KN> struct ProjTile {
     typedef GemmCfg<T, 256, BN, 4, BN == 128 ? 3 : 2, KN> C;
 };
 
+// Tiles of small problems (16-bit weights in [N][K]): fewer rows and columns,
+// so that a launch fills the CUs, and two workgroups per CU.  The K order of an
+// output is the same in every tile, and so is the result bit for bit.
+template <typename T> struct Tile64x64 { typedef GemmCfg<T, 64, 64, 4, 4, false> C; };
+template <typename T> struct Tile128x64 { typedef GemmCfg<T, 128, 64, 4, 3, false> C; };
+template <typename T> struct Tile128x128 { typedef GemmCfg<T, 128, 128, 2, 2, false> C; };
+
 template <typename C>
 int launch_cfg(GemmParams p, bool bias, hipStream_t stream) {
     p.tiles_m = (p.M + C::BM - 1) / C::BM;
@@ -170,12 +177,45 @@ inline int pick_bn(int M, int N, const int* cands, int n_cands) {
     return best;
 }
 
+// Tile for 16-bit weights in [N][K]: a BN of the 256-row tiles, or one of the
+// small tiles (ids 1-3).  Costs are microseconds per 64-deep K stage, measured
+// on MI355X: a round of 256-row tiles (BN + 92) x 0.0047 (pick_bn's model); a
+// small tile c1 alone on its CU and c2 for the two a CU holds.  Measured (bf16,
+// us, the 256-row choice against this one): M=1024, N=3456, K=1152 21.9 -> 14.9
+// (128x128); M=1024, N=1152, K=1152 20.7 -> 10.7 (128x64); M=577, N=704, K=704
+// 14.2 -> 6.9 (64x64); M=3220, N=1152, K=384 10.7 -> 7.6; M=2048, N=2240,
+// K=2240 36.5 -> 33.5; and where it keeps the 256-row tile: M=4096, N=3456,
+// K=1152 34.5 against 37.2, M=2048, N=6720, K=2240 57.9 against 68.0.
+inline int pick_tile(int M, int N) {
+    static const int cands[] = {320, 224, 256, 192, 160, 128};
+    const long long cus = device_cu_count();
+    int best = pick_bn(M, N, cands, 6);
+    const long long big = (long long)((M + 255) / 256) * ((N + best - 1) / best);
+    double best_cost = (double)((big + cus - 1) / cus) * (best + 92) * 0.0047;
+    struct Small { int bm, bn; double c1, c2; };
+    static const Small small[] = {{64, 64, 0.32, 0.46}, {128, 64, 0.40, 0.70}, {128, 128, 0.61, 1.02}};
+    for (int i = 0; i < 3; ++i) {
+        const long long n = (long long)((M + small[i].bm - 1) / small[i].bm) * ((N + small[i].bn - 1) / small[i].bn);
+        const long long rest = n % (2 * cus);
+        const double cost = (double)(n / (2 * cus)) * small[i].c2 + (rest == 0 ? 0 : rest <= cus ? small[i].c1 : small[i].c2);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = i + 1;
+        }
+    }
+    return best;
+}
+
+// tile: an id or width of pick_tile, 0 = chosen per shape.
 template <typename T, bool KN>
-int launch_gemm(const GemmParams& p, bool bias, hipStream_t st) {
-    // 16-bit weights in [N][K]: six widths; fp32 or WeightT: 256 and 128.
+int launch_gemm(const GemmParams& p, bool bias, hipStream_t st, int tile) {
+    // 16-bit weights in [N][K]: six widths and three small tiles; fp32 or
+    // WeightT: 256 and 128.
     if constexpr (sizeof(T) == 2 && !KN) {
-        static const int cands[] = {320, 224, 256, 192, 160, 128};
-        switch (pick_bn(p.M, p.N, cands, 6)) {
+        switch (tile ? tile : pick_tile(p.M, p.N)) {
+        case 1: return launch_cfg<typename Tile64x64<T>::C>(p, bias, st);
+        case 2: return launch_cfg<typename Tile128x64<T>::C>(p, bias, st);
+        case 3: return launch_cfg<typename Tile128x128<T>::C>(p, bias, st);
         case 320: return launch_cfg<typename ProjTile<T, 320, KN>::C>(p, bias, st);
         case 256: return launch_cfg<typename ProjTile<T, 256, KN>::C>(p, bias, st);
         case 224: return launch_cfg<typename ProjTile<T, 224, KN>::C>(p, bias, st);
@@ -190,8 +230,8 @@ int launch_gemm(const GemmParams& p, bool bias, hipStream_t st) {
     }
 }
 
-template <typename T> int launch_gemm_layout(const GemmParams& p, int layout, bool bias, hipStream_t st) {
-    return layout == KF_WEIGHT_NK ? launch_gemm<T, false>(p, bias, st) : launch_gemm<T, true>(p, bias, st);
+template <typename T> int launch_gemm_layout(const GemmParams& p, int layout, bool bias, hipStream_t st, int tile) {
+    return layout == KF_WEIGHT_NK ? launch_gemm<T, false>(p, bias, st, tile) : launch_gemm<T, true>(p, bias, st, 0);
 }
 
 bool aligned(const void* p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
@@ -199,10 +239,10 @@ bool aligned(const void* p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 }  // namespace
 }  // namespace kf
 
-extern "C" int kf_proj_gemm(const void* x, const void* weight, const void* bias, void* y, int64_t m, int64_t n,
-                            int64_t k, int64_t ldx, int64_t ldy, int weight_layout, int dtype,
-                            kf_stream_t stream) {
-    using namespace kf;
+namespace kf {
+namespace {
+int proj_gemm_run(const void* x, const void* weight, const void* bias, void* y, int64_t m, int64_t n, int64_t k,
+                  int64_t ldx, int64_t ldy, int weight_layout, int dtype, int tile, kf_stream_t stream) {
     clear_error();
     KF_REQUIRE(dtype == KF_BF16 || dtype == KF_F16 || dtype == KF_F32, KF_E_INVALID,
                "kf_proj_gemm: dtype must be bf16, f16 or f32");
@@ -233,7 +273,24 @@ extern "C" int kf_proj_gemm(const void* x, const void* weight, const void* bias,
     p.staged_out = aligned(y, 16) && (ldy * es) % 16 == 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool b = bias != nullptr;
-    if (dtype == KF_BF16) return launch_gemm_layout<bf16>(p, weight_layout, b, st);
-    if (dtype == KF_F16) return launch_gemm_layout<f16>(p, weight_layout, b, st);
-    return launch_gemm_layout<float>(p, weight_layout, b, st);
+    if (dtype == KF_BF16) return launch_gemm_layout<bf16>(p, weight_layout, b, st, tile);
+    if (dtype == KF_F16) return launch_gemm_layout<f16>(p, weight_layout, b, st, tile);
+    return launch_gemm_layout<float>(p, weight_layout, b, st, tile);
+}
+}  // namespace
+}  // namespace kf
+
+extern "C" int kf_proj_gemm(const void* x, const void* weight, const void* bias, void* y, int64_t m, int64_t n,
+                            int64_t k, int64_t ldx, int64_t ldy, int weight_layout, int dtype,
+                            kf_stream_t stream) {
+    return kf::proj_gemm_run(x, weight, bias, y, m, n, k, ldx, ldy, weight_layout, dtype, 0, stream);
+}
+
+// Test entry point (not in the public header): kf_proj_gemm with the output
+// tile forced (16-bit types in the KF_WEIGHT_NK layout: 1 = 64x64, 2 = 128x64,
+// 3 = 128x128, 128..320 = that width of the 256-row tile, 0 = chosen per shape).
+extern "C" int kfm_proj_gemm_tile(const void* x, const void* weight, const void* bias, void* y, int64_t m, int64_t n,
+                                  int64_t k, int64_t ldx, int64_t ldy, int weight_layout, int dtype, int tile,
+                                  kf_stream_t stream) {
+    return kf::proj_gemm_run(x, weight, bias, y, m, n, k, ldx, ldy, weight_layout, dtype, tile, stream);
 }
