@@ -162,6 +162,11 @@ int64_t kf_linattn_workspace_bytes(int64_t batch, int64_t heads, int64_t dim,
  */
 int kf_linattn_workspace_init(void* workspace, int64_t workspace_bytes, kf_stream_t stream);
 
+/* Bytes at the start of the workspace that a call of this shape needs zero on
+ * entry (0 for shapes without cross-workgroup counters): what a caller that
+ * zeroes the workspace before every call passes to kf_linattn_workspace_init. */
+int64_t kf_linattn_control_bytes(int64_t batch, int64_t heads, int64_t dim);
+
 /*
  * out[b, n, h*D + r] = sum_c S[r][c] relu(q)[n,c] / (sum_c z[c] relu(q)[n,c] + eps)
  * with S = sum_n v[n,:]^T relu(k)[n,:] and z = sum_n relu(k)[n,:] per (b, h),
@@ -273,6 +278,17 @@ int kf_linattn_noalloc_check(kf_stream_t stream);
 int kf_rope_packed(void* qkv, const float* cos, const float* sin,
                    int64_t batch, int64_t seq_len, int64_t heads, int64_t dim,
                    int dtype, kf_stream_t stream);
+
+/*
+ * LiteLA's q/k norm (kf_rmsnorm_fwd_strided on the q and the k rows, with
+ * weights of heads * dim elements in qkv's dtype) and, when cos and sin are not
+ * NULL, kf_rope_packed, in one pass over the packed qkv; the same results bit
+ * for bit.  Rows of whole 16-byte vectors up to 16 KiB (KF_E_UNSUPPORTED
+ * otherwise); every buffer 16-byte aligned.
+ */
+int kf_qk_norm_rope(void* qkv, const void* q_weight, const void* k_weight, const float* cos, const float* sin,
+                    int64_t batch, int64_t seq_len, int64_t heads, int64_t dim, float eps, int dtype,
+                    kf_stream_t stream);
 
 /* ------------------------------------------------------------------ */
 /* SANA projections                                                    */

@@ -52,9 +52,10 @@ _ws_lock = threading.Lock()
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 
-def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
+def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int]) -> torch.Tensor:
     """The zero-initialised workspace of the current stream on `device`, at
-    least `nbytes` long (its control words are zero between calls).
+    least `nbytes` long (its control words are zero between calls); ``shape``
+    is the call's (batch, heads, dim).
 
     Under graph capture the zeroing is recorded with every call instead: the
     fill of a fresh tensor would only run when the graph that happened to
@@ -70,8 +71,11 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
             ws = make(max(nbytes, 1 << 20), device=device, dtype=torch.uint8)
             _workspaces[key] = ws
     if capturing:
-        rc = _lib.load().kf_linattn_workspace_init(_lib.ptr(ws), ws.numel(), ctypes.c_void_p(stream.cuda_stream))
-        _lib.check(rc, "kf_linattn_workspace_init")
+        lib = _lib.load()
+        control = lib.kf_linattn_control_bytes(*shape)
+        if control:
+            rc = lib.kf_linattn_workspace_init(_lib.ptr(ws), control, ctypes.c_void_p(stream.cuda_stream))
+            _lib.check(rc, "kf_linattn_workspace_init")
     return ws
 
 
@@ -106,7 +110,7 @@ def _launch(kind: str, qkv: torch.Tensor, out: torch.Tensor, B: int, N: int, hea
     # unit), so a larger request needs no larger workspace.
     ws_splits = min(splits, max(1, -(-N // 32)))
     ws_bytes = int(lib.kf_linattn_workspace_bytes(B, heads, dim, ws_splits))
-    ws = _workspace(qkv.device, ws_bytes)
+    ws = _workspace(qkv.device, ws_bytes, (B, heads, dim))
     stream = _lib.stream_of(qkv)
     if kind == "fwd":
         rc = lib.kf_linattn_fwd(_lib.ptr(qkv), _lib.ptr(out), _lib.ptr(ws), ws.numel(), B, N, heads, dim,

@@ -27,10 +27,10 @@ Otherwise (unfused):
 1. ``qkv = x @ Wqkv^T (+ b)`` -- the hand-written MFMA GEMM (``kf_proj_gemm``,
    projection.py) on the module's ``[3C, C]`` weight, into the packed
    ``[B, N, 3, C]`` layout.
-2. ``qk_norm``: RMSNorm over the C channels of each token's q and k, in place
-   in the packed buffer (``kf_rmsnorm_fwd_strided``, no copies).
-3. ``rotary_emb = (cos, sin)``: rotary embedding of q and k, in place in the
-   packed buffer (``kf_rope_packed``; original.py:136-138).
+2. ``qk_norm``: RMSNorm over the C channels of each token's q and k, and
+3. ``rotary_emb = (cos, sin)``: rotary embedding of q and k (original.py:
+   136-138), in place in the packed buffer: one pass (``kf_qk_norm_rope``)
+   with the norm, ``kf_rope_packed`` without it.
 4. ReLU linear attention (``kf_linattn_fwd``: split states on MFMA, fixed-order
    split reduction, MFMA output contraction), fp32 arithmetic.
 5. ``y = out @ Wproj^T + b`` -- the same GEMM with the bias in its epilogue.
@@ -96,35 +96,51 @@ def apply_rotary_emb(x: torch.Tensor, freqs_cis, use_real: bool = True, use_real
     return torch.stack((re, im), dim=stack_dim).flatten(*flat).to(x.dtype)
 
 
-def _project_qkv(x: torch.Tensor, weight: torch.Tensor, bias, q_norm_weight, k_norm_weight,
-                 norm_eps: float) -> torch.Tensor:
-    """``x[B, N, C] -> qkv[B, N, 3, C]``: the MFMA projection GEMM, then the
-    optional q/k RMSNorm over C in place in the packed buffer (original.py:122-130)."""
-    B, N, C = x.shape
-    qkv = linear(x, weight.detach(), None if bias is None else bias.detach()).reshape(B, N, 3, C)
+def _norm_rotate_(qkv: torch.Tensor, heads: int, dim: int, q_norm_weight, k_norm_weight, norm_eps: float,
+                  tables) -> None:
+    """The optional q/k RMSNorm over C and rotary embedding, in place in the
+    packed ``qkv[B, N, 3, C]`` (original.py:122-138): one pass over q and k
+    (``kf_qk_norm_rope``) where there is a norm and its layout allows, the
+    kernels of each step otherwise.  ``tables`` is the fp32 (cos, sin) pair or
+    None."""
+    B, N, _, C = qkv.shape
+    lib = _lib.load()
+    cos, sin = tables if tables is not None else (None, None)
     if q_norm_weight is not None:
-        rms_norm_rows_(qkv[:, :, 0], q_norm_weight.detach().to(qkv.dtype), norm_eps)
-        rms_norm_rows_(qkv[:, :, 1], k_norm_weight.detach().to(qkv.dtype), norm_eps)
-    return qkv
+        qw, kw = (w.detach().to(qkv.dtype).contiguous() for w in (q_norm_weight, k_norm_weight))
+        row_bytes = C * qkv.element_size()
+        one_pass = (0 < row_bytes <= 16384 and row_bytes % 16 == 0 and qw.numel() == kw.numel() == C
+                    and (cos is None or dim % 8 == 0)
+                    and all(t is None or t.data_ptr() % 16 == 0 for t in (qkv, qw, kw, cos, sin)))
+        if one_pass:
+            rc = lib.kf_qk_norm_rope(_lib.ptr(qkv), _lib.ptr(qw), _lib.ptr(kw), _lib.ptr(cos), _lib.ptr(sin), B, N,
+                                     heads, dim, float(norm_eps), _lib.kf_dtype(qkv.dtype), _lib.stream_of(qkv))
+            _lib.check(rc, "kf_qk_norm_rope")
+            return
+        rms_norm_rows_(qkv[:, :, 0], qw, norm_eps)
+        rms_norm_rows_(qkv[:, :, 1], kw, norm_eps)
+    if cos is not None:
+        rc = lib.kf_rope_packed(_lib.ptr(qkv), _lib.ptr(cos), _lib.ptr(sin), B, N, heads, dim,
+                                _lib.kf_dtype(qkv.dtype), _lib.stream_of(qkv))
+        _lib.check(rc, "kf_rope_packed")
 
 
 def _attention_output(x: torch.Tensor, qkv_weight: torch.Tensor, qkv_bias, q_norm_weight, k_norm_weight,
                       norm_eps: float, heads: int, dim: int, eps: float, fused: Optional[bool],
-                      rotary_fn=None) -> torch.Tensor:
+                      tables=None) -> torch.Tensor:
     """LiteLA's attention output before the output projection.  Without q/k
     norm and rotary embedding, with head dim 32 and a 16-bit dtype, the fused
     projection + attention kernels (fused.py) run when ``fused`` is True, or
     when it is None and they pay for the shape; otherwise the projection GEMM
     fills the packed qkv, the optional norm and rotation run in place, and the
     linear-attention kernel follows."""
-    B, N, _ = x.shape
-    if q_norm_weight is None and rotary_fn is None and fused_applicable(x.dtype, dim):
+    B, N, C = x.shape
+    if q_norm_weight is None and tables is None and fused_applicable(x.dtype, dim):
         if fused if fused is not None else prefer_fused(B, N, heads, x.device):
             return litela_fused_attention(x, qkv_weight.detach(),
                                           None if qkv_bias is None else qkv_bias.detach(), heads, eps)
-    qkv = _project_qkv(x, qkv_weight, qkv_bias, q_norm_weight, k_norm_weight, norm_eps)
-    if rotary_fn is not None:
-        rotary_fn(qkv)
+    qkv = linear(x, qkv_weight.detach(), None if qkv_bias is None else qkv_bias.detach()).reshape(B, N, 3, C)
+    _norm_rotate_(qkv, heads, dim, q_norm_weight, k_norm_weight, norm_eps, tables)
     # The kernel rounds its fp32 result straight to x's dtype (round to
     # nearest even), as `.to(dtype)` on the fp32 result would.
     return linear_attention(qkv, heads, dim, eps, x.dtype)
@@ -216,21 +232,19 @@ class LiteLA(nn.Module):
 
     def _attn_out(self, x: torch.Tensor, rotary_emb=None) -> torch.Tensor:
         qn, kn, norm_eps = self._norm_weights()
-        rot = None if rotary_emb is None else (lambda qkv: self._rotate_(qkv, rotary_emb))
+        tables = None if rotary_emb is None else self._rotary_tables(x, rotary_emb)
         return _attention_output(x, self.qkv.weight, self.qkv.bias, qn, kn, norm_eps, self.heads, self.dim,
-                                 self.eps, self.fused_projection, rot)
+                                 self.eps, self.fused_projection, tables)
 
-    def _rotate_(self, qkv: torch.Tensor, rotary_emb) -> None:
-        """q and k of the packed qkv rotated in place (original.py:136-138)."""
-        B, N, _, C = qkv.shape
+    def _rotary_tables(self, x: torch.Tensor, rotary_emb):
+        """The fp32 (cos, sin) tables ``[N, head_dim]`` on x's device (original.py:136-138)."""
+        N = x.shape[1]
         if not isinstance(rotary_emb, (tuple, list)) or len(rotary_emb) != 2:
             raise ValueError("rotary_emb must be a (cos, sin) pair of [N, head_dim] tensors")
-        cos, sin = (t.detach().to(device=qkv.device, dtype=torch.float32).contiguous() for t in rotary_emb)
+        cos, sin = (t.detach().to(device=x.device, dtype=torch.float32).contiguous() for t in rotary_emb)
         if cos.shape != (N, self.dim) or sin.shape != (N, self.dim):
             raise ValueError(f"rotary_emb tensors must be [{N}, {self.dim}], got {tuple(cos.shape)}, {tuple(sin.shape)}")
-        rc = _lib.load().kf_rope_packed(_lib.ptr(qkv), _lib.ptr(cos), _lib.ptr(sin), B, N, self.heads, self.dim,
-                                        _lib.kf_dtype(qkv.dtype), _lib.stream_of(qkv))
-        _lib.check(rc, "kf_rope_packed")
+        return cos, sin
 
     def forward(self, x: torch.Tensor, mask=None, HW=None, rotary_emb=None, block_id=None,
                 block_mask=None) -> torch.Tensor:

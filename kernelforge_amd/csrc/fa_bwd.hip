@@ -336,7 +336,7 @@ void fa_bwd_dq_kernel(const FaBwdParams p) {
 // wavefront, scanning query tiles of FaTile::BK rows of every query head of
 // the group.
 // ---------------------------------------------------------------------------
-template <typename T, int DP>
+template <typename T, int DP, bool SPLIT>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
 void fa_bwd_dkdv_kernel(const FaBwdParams p) {
@@ -370,11 +370,13 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
 
     // Causal runs of a split key tile differ in length: longest first.
     const int xlogical = xcd_logical_block();
-    const int logical = p.causal && p.ksplits > 1 ? causal_tile_order(xlogical, p.n_ktiles) : xlogical;
+    const int logical = SPLIT && p.causal ? causal_tile_order(xlogical, p.n_ktiles) : xlogical;
     const int ktile = logical % p.n_ktiles;
-    int rest = logical / p.n_ktiles;
-    const int split = rest % p.ksplits;
-    rest /= p.ksplits;
+    int rest = logical / p.n_ktiles, split = 0;
+    if constexpr (SPLIT) {
+        split = rest % p.ksplits;
+        rest /= p.ksplits;
+    }
     const int hk = rest % p.Hkv, b = rest / p.Hkv;
 
     const int k0 = ktile * kBKEYS;             // first key of the workgroup
@@ -401,10 +403,14 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
     const int n_rt = (p.Nq + kBR - 1) / kBR;
     const int rt0 = p.causal ? min(n_rt, max(0, k0 - diag) / kBR) : 0;
     const int per_head = n_rt - rt0;
-    // This workgroup's run of the (head, row tile) sequence.
-    const int per_split = (per_head * p.group + p.ksplits - 1) / p.ksplits;
-    const int u0 = min(per_head * p.group, split * per_split);
-    const int ntiles = min(per_head * p.group, u0 + per_split);
+    // This workgroup's run of the (head, row tile) sequence (SPLIT: one of
+    // p.ksplits).
+    int u0 = 0, ntiles = per_head * p.group;
+    if constexpr (SPLIT) {
+        const int per_split = (ntiles + p.ksplits - 1) / p.ksplits;
+        u0 = min(ntiles, split * per_split);
+        ntiles = min(ntiles, u0 + per_split);
+    }
     const float c = p.scale_log2;
 
     const uint32_t voff = full_tile_shortcut<DP>() ? full_tile_lane_offset<T, DP>(q_row_stride, wave, lane) : 0u;
@@ -547,7 +553,7 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
         if (u + 1 < ntiles) step(u + 1, std::integral_constant<int, 1>{});
     }
 
-    if (p.ksplits > 1) {
+    if constexpr (SPLIT) {
         const int64_t part = split * ((int64_t)p.B * p.Nk * kv_row_stride) + kv_off;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
@@ -601,7 +607,7 @@ void fa_bwd_dkdv_kernel(const FaBwdParams p) {
 template <int DP> constexpr int dkdv_wide_blocks() { return DP <= 32 ? 4 : 2; }
 template <int DP> constexpr int dkdv_wide_keys() { return 16 * FaTile<DP>::WAVES * dkdv_wide_blocks<DP>(); }
 
-template <typename T, int DP>
+template <typename T, int DP, bool SPLIT>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
 void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
@@ -639,9 +645,11 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
     const int n_kt = (p.Nk + kBKEYS - 1) / kBKEYS;
     const int logical = p.causal ? causal_tile_order(xcd_logical_block(), n_kt) : xcd_logical_block();
     const int ktile = logical % n_kt;
-    int rest = logical / n_kt;
-    const int split = rest % p.ksplits;
-    rest /= p.ksplits;
+    int rest = logical / n_kt, split = 0;
+    if constexpr (SPLIT) {
+        split = rest % p.ksplits;
+        rest /= p.ksplits;
+    }
     const int hk = rest % p.Hkv, b = rest / p.Hkv;
 
     const int k0 = ktile * kBKEYS;  // first key of the workgroup
@@ -675,10 +683,14 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
     const int n_rt = (p.Nq + kBR - 1) / kBR;
     const int rt0 = p.causal ? min(n_rt, max(0, k0 - diag) / kBR) : 0;
     const int per_head = n_rt - rt0;
-    // This workgroup's run of the (head, row tile) sequence.
-    const int per_split = (per_head * p.group + p.ksplits - 1) / p.ksplits;
-    const int u0 = min(per_head * p.group, split * per_split);
-    const int ntiles = min(per_head * p.group, u0 + per_split);
+    // This workgroup's run of the (head, row tile) sequence (SPLIT: one of
+    // p.ksplits).
+    int u0 = 0, ntiles = per_head * p.group;
+    if constexpr (SPLIT) {
+        const int per_split = (ntiles + p.ksplits - 1) / p.ksplits;
+        u0 = min(ntiles, split * per_split);
+        ntiles = min(ntiles, u0 + per_split);
+    }
     const float c = p.scale_log2;
 
     const uint32_t voff = panel_lane_offset<T>(q_row_stride, lane);
@@ -855,7 +867,7 @@ void fa_bwd_dkdv_wide_kernel(const FaBwdParams p) {
     for (int kb = 0; kb < KB; ++kb) {
         const int kr = k0w + 16 * kb + (lane_out & 15);
         const int64_t kv_off = kv_base + (int64_t)kr * kv_row_stride;
-        if (p.ksplits > 1) {
+        if constexpr (SPLIT) {
             const int64_t part = split * ((int64_t)p.B * p.Nk * kv_row_stride) + kv_off;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
@@ -1030,18 +1042,24 @@ int launch_bwd(FaBwdParams p, const FaBwdPlan& plan, hipStream_t stream) {
         if (int rc = check_launch("fa_bwd_dq_kernel launch")) return rc;
     }
     if (kblocks == 0) return KF_OK;
+    const dim3 kgrid((unsigned)kblocks);
     bool launched = false;
     if constexpr (DP <= 128) {
         if (plan.wide) {
-            hipLaunchKernelGGL((fa_bwd_dkdv_wide_kernel<T, DP>), dim3((unsigned)kblocks), threads, 0, stream, p);
-            if (int rc = check_launch("fa_bwd_dkdv_wide_kernel launch")) return rc;
+            if (p.ksplits > 1)
+                hipLaunchKernelGGL((fa_bwd_dkdv_wide_kernel<T, DP, true>), kgrid, threads, 0, stream, p);
+            else
+                hipLaunchKernelGGL((fa_bwd_dkdv_wide_kernel<T, DP, false>), kgrid, threads, 0, stream, p);
             launched = true;
         }
     }
     if (!launched) {
-        hipLaunchKernelGGL((fa_bwd_dkdv_kernel<T, DP>), dim3((unsigned)kblocks), threads, 0, stream, p);
-        if (int rc = check_launch("fa_bwd_dkdv_kernel launch")) return rc;
+        if (p.ksplits > 1)
+            hipLaunchKernelGGL((fa_bwd_dkdv_kernel<T, DP, true>), kgrid, threads, 0, stream, p);
+        else
+            hipLaunchKernelGGL((fa_bwd_dkdv_kernel<T, DP, false>), kgrid, threads, 0, stream, p);
     }
+    if (int rc = check_launch("fa_bwd_dkdv_kernel launch")) return rc;
     if (p.ksplits == 1) return KF_OK;
     const int64_t n4 = (int64_t)p.B * p.Nk * p.Hkv * p.D / 4;
     if ((n4 + 255) / 256 > 0x7fffff) {

@@ -1199,6 +1199,13 @@ extern "C" int64_t kf_linattn_workspace_bytes(int64_t batch, int64_t heads, int6
     return kf::kCtrlBytes + (int64_t)sizeof(float) * batch * heads * state * (splits + 1);
 }
 
+extern "C" int64_t kf_linattn_control_bytes(int64_t batch, int64_t heads, int64_t dim) {
+    if (batch <= 0 || heads <= 0 || dim != kf::kD) return 0;  // only the one-launch kernel has group counters
+    const int64_t groups = batch * ((heads + 1) / 2);
+    return 4 * (int64_t)(kf::kCtrlHeader +
+                         kf::kCtrlStride * (groups < kf::kMaxGroupsPerLaunch ? groups : kf::kMaxGroupsPerLaunch));
+}
+
 extern "C" int kf_linattn_workspace_init(void* workspace, int64_t workspace_bytes, kf_stream_t stream) {
     using namespace kf;
     KF_REQUIRE(workspace_bytes >= 0, KF_E_INVALID, "linattn: negative workspace size");

@@ -20,6 +20,9 @@
 // stage the weight in LDS once per block: re-reading it from L2 for every row
 // cost 2-3% of the HBM rate at 2048-4096 channels; with one row per block
 // (8192) the staging costs more than it saves.
+#include <initializer_list>
+#include <type_traits>
+
 #include "kf_common.h"
 
 namespace kf {
@@ -160,6 +163,141 @@ __global__ __launch_bounds__(64 * WAVES) void rmsnorm_vec_kernel(const TX* x, co
             store_nt(yr + j, ov);
         }
     }
+}
+
+// LiteLA's q/k norm and rotary embedding in one pass, in place on the packed
+// qkv[token][q, k, v][dim]: the arithmetic of
+// rmsnorm_vec_kernel, with its layout and so its bits, then that of
+// rope_packed_kernel on the rounded result (channel pairs lie within a
+// 16-byte vector, a vector within a head).  HBM bound: it reads and writes q
+// and k once, where two norm launches and a rotary one did so twice.  Measured
+// on MI355X at 8192 tokens of 2240 channels, bf16 (147 MB): 40 us with the
+// rotary embedding against 62 for the three launches, 37 without it against 36
+// for two (which a small call pays for twice: 7 against 20 us at 1024 x 1152).
+// Staging the weight in LDS, or q rows and k rows in separate halves of the
+// grid, was no faster; requesting the weight and table values with the row,
+// per vector, was slower (53 us).
+// ROPE: 0 = norm only, 1 = a head divides the 64 vectors of a load (D = 8..512,
+// powers of two), so that a lane meets the same table values in every vector and
+// loads them once, 2 = any D.
+template <typename T, int VPT, int WPR, int WAVES, int ROPE>
+__global__ __launch_bounds__(64 * WAVES) void rmsnorm_qk_kernel(T* qkv, const T* __restrict__ qw,
+                                                                const T* __restrict__ kw,
+                                                                const float* __restrict__ cs,
+                                                                const float* __restrict__ sn, int64_t tokens,
+                                                                int64_t N, int dim, int D, float eps) {
+    // The rotary products and their sum are rounded one by one (rope.hip).
+#pragma clang fp contract(off)
+    constexpr int VEC = 16 / sizeof(T);
+    typedef Pack<T, VEC> P;
+    constexpr int RPB = WAVES / WPR;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int slot = wave / WPR, slice = wave % WPR;
+    const int64_t r = (int64_t)blockIdx.x * RPB + slot;  // a token's q row, then its k row
+    const int64_t tok = r >> 1;
+    const int part_k = (int)(r & 1);
+    const bool ok = tok < tokens;
+    const int nvec = dim / VEC;
+    const P* wr = reinterpret_cast<const P*>(part_k ? kw : qw);
+    P* row = reinterpret_cast<P*>(qkv + (tok * 3 + part_k) * (int64_t)dim);
+
+    typedef Pack<float, VEC> F;
+    P xv[VPT];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int j = (i * WPR + slice) * 64 + lane;
+        xv[i] = ok && j < nvec ? load_nt(row + j) : P{};
+    }
+    const int64_t trow = tok % N * D;
+    F cv, sv;
+    if constexpr (ROPE == 1) {
+        cv = *reinterpret_cast<const F*>(cs + trow + lane * VEC % D);
+        sv = *reinterpret_cast<const F*>(sn + trow + lane * VEC % D);
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            const float f = to_f32(xv[i].v[k]);
+            ss = fmaf(f, f, ss);
+        }
+    ss = wave_sum(ss);
+    if constexpr (WPR > 1) {
+        __shared__ float part[WAVES];
+        if (lane == 0) part[wave] = ss;
+        __syncthreads();
+        float t = 0.f;
+#pragma unroll
+        for (int s = 0; s < WPR; ++s) t += part[slot * WPR + s];
+        ss = t;
+    }
+    if (!ok) return;
+    const float inv = 1.0f / sqrtf(ss / (float)dim + eps);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int j = (i * WPR + slice) * 64 + lane;
+        if (j < nvec) {
+            const P wv = wr[j];
+            P ov;
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                // The product is rounded to fp32 first, as rmsnorm_vec_kernel
+                // does; left to itself the compiler forms v_fma_mixlo_f16 for
+                // some of them, which rounds once.
+                float t = to_f32(xv[i].v[k]) * inv;
+                if constexpr (__is_same(T, f16)) asm("" : "+v"(t));
+                ov.v[k] = from_f32<T>(to_f32(from_f32<T>(t)) * to_f32(wv.v[k]));
+            }
+            if constexpr (ROPE == 2) {
+                cv = *reinterpret_cast<const F*>(cs + trow + j * VEC % D);
+                sv = *reinterpret_cast<const F*>(sn + trow + j * VEC % D);
+            }
+            if constexpr (ROPE != 0) {
+#pragma unroll
+                for (int k = 0; k < VEC; k += 2) {
+                    const float re = to_f32(ov.v[k]), im = to_f32(ov.v[k + 1]);
+                    const float a0 = re * cv.v[k], b0 = -im * sv.v[k];
+                    const float a1 = im * cv.v[k + 1], b1 = re * sv.v[k + 1];
+                    ov.v[k] = from_f32<T>(a0 + b0);
+                    ov.v[k + 1] = from_f32<T>(a1 + b1);
+                }
+            }
+            store_nt(row + j, ov);
+        }
+    }
+}
+
+template <typename T, int VPT, int WPR, int WAVES>
+int launch_qk(void* qkv, const void* qw, const void* kw, const float* cs, const float* sn, int64_t tokens, int64_t N,
+              int64_t dim, int64_t D, float eps, hipStream_t stream) {
+    const int64_t blocks = (2 * tokens + WAVES / WPR - 1) / (WAVES / WPR);
+    KF_REQUIRE(blocks <= 0x7fffff, KF_E_UNSUPPORTED, "qk_norm: %lld tokens exceed the grid limit", (long long)tokens);
+    const dim3 grid((unsigned)blocks);
+    auto launch = [&](auto ropec) {
+        hipLaunchKernelGGL((rmsnorm_qk_kernel<T, VPT, WPR, WAVES, decltype(ropec)::value>), grid, dim3(64 * WAVES), 0,
+                           stream, static_cast<T*>(qkv), static_cast<const T*>(qw), static_cast<const T*>(kw), cs, sn,
+                           tokens, N, (int)dim, (int)D, eps);
+    };
+    if (!cs) launch(std::integral_constant<int, 0>{});
+    else if (64 * (16 / (int)sizeof(T)) % D == 0) launch(std::integral_constant<int, 1>{});
+    else launch(std::integral_constant<int, 2>{});
+    return check_launch("rmsnorm_qk_kernel launch");
+}
+
+template <typename T>
+int dispatch_qk(void* qkv, const void* qw, const void* kw, const float* cs, const float* sn, int64_t tokens,
+                int64_t N, int64_t dim, int64_t D, float eps, hipStream_t stream) {
+    const int64_t nvec = dim / (16 / (int64_t)sizeof(T));
+#define KF_RMS_QK(VPT, WPR, WAVES) \
+    return launch_qk<T, VPT, WPR, WAVES>(qkv, qw, kw, cs, sn, tokens, N, dim, D, eps, stream)
+    // The shapes of dispatch() above, whose sums these must equal.
+    if (nvec <= 64) KF_RMS_QK(1, 1, 4);
+    if (nvec <= 128) KF_RMS_QK(2, 1, 4);
+    if (nvec <= 256) KF_RMS_QK(2, 2, 4);
+    if (nvec <= 512) KF_RMS_QK(2, 4, 8);
+    KF_RMS_QK(2, 8, 8);
+#undef KF_RMS_QK
 }
 
 // Any dim / alignment: one block per row, two passes over the row.
@@ -622,6 +760,31 @@ extern "C" int kf_rmsnorm_fwd_strided(const void* x, const void* weight, void* y
     KF_REQUIRE(valid_dt(dtype), KF_E_INVALID, "rmsnorm: unknown dtype %d", dtype);
     return by_types<FwdOp>(dtype, dtype, x, weight, y, rows, dim, ld_x, ld_y, eps,
                            static_cast<hipStream_t>(stream));
+}
+
+extern "C" int kf_qk_norm_rope(void* qkv, const void* q_weight, const void* k_weight, const float* cos,
+                               const float* sin, int64_t batch, int64_t seq_len, int64_t heads, int64_t dim,
+                               float eps, int dtype, kf_stream_t stream) {
+    using namespace kf;
+    KF_REQUIRE(batch >= 0 && seq_len >= 0 && heads > 0 && dim > 0, KF_E_INVALID, "qk_norm: bad shape");
+    KF_REQUIRE(valid_dt(dtype), KF_E_INVALID, "qk_norm: unknown dtype %d", dtype);
+    KF_REQUIRE(heads <= (1 << 20) && dim <= 4096 && batch <= (1 << 20) && seq_len <= ((int64_t)1 << 31), KF_E_INVALID,
+               "qk_norm: shape out of range");
+    const int64_t C = heads * dim, es = dtype == KF_F32 ? 4 : 2;
+    KF_REQUIRE((cos == nullptr) == (sin == nullptr), KF_E_INVALID, "qk_norm: cos and sin come together");
+    KF_REQUIRE(C * es % 16 == 0 && C * es <= 16384 && (!cos || dim % 8 == 0), KF_E_UNSUPPORTED,
+               "qk_norm: rows must be whole 16-byte vectors, at most 16 KiB, and rotated heads whole multiples of 8");
+    if (batch == 0 || seq_len == 0) return KF_OK;
+    KF_REQUIRE(qkv && q_weight && k_weight, KF_E_INVALID, "qk_norm: null pointer");
+    for (const void* p : {(const void*)qkv, q_weight, k_weight, (const void*)cos, (const void*)sin})
+        KF_REQUIRE(aligned_to(p, 16), KF_E_INVALID, "qk_norm: buffers must be 16-byte aligned");
+    const int64_t tokens = batch * seq_len;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (dtype) {
+        case KF_F32: return dispatch_qk<float>(qkv, q_weight, k_weight, cos, sin, tokens, seq_len, C, dim, eps, s);
+        case KF_F16: return dispatch_qk<f16>(qkv, q_weight, k_weight, cos, sin, tokens, seq_len, C, dim, eps, s);
+        default: return dispatch_qk<bf16>(qkv, q_weight, k_weight, cos, sin, tokens, seq_len, C, dim, eps, s);
+    }
 }
 
 extern "C" int kf_rmsnorm_fwd(const void* x, const void* weight, void* y, int64_t rows,
