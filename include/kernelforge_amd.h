@@ -403,6 +403,15 @@ int kf_fa_jvp(const void* q, const void* k, const void* v,
               int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
               int64_t D, float scale, int causal, int dtype, kf_stream_t stream);
 
+/* The same with a workspace (see kf_fa_fwd_ws). */
+int64_t kf_fa_jvp_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                                  int causal);
+int kf_fa_jvp_ws(const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                 const void* tv, const void* o, const float* lse, void* to,
+                 void* workspace, int64_t workspace_bytes,
+                 int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                 float scale, int causal, int dtype, kf_stream_t stream);
+
 /*
  * Fused single pass: O, LSE and tO in one scan over the K/V tiles with the
  * online recurrences of flash-attention-jvp-derivation.md:388-558

@@ -99,6 +99,12 @@ SIGNATURES = {
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
          _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
     ),
+    "kf_fa_jvp_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
+    "kf_fa_jvp_ws": (
+        _int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _c_void_p],
+    ),
     "kf_fa_bwd_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
     "kf_fa_bwd_split_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
     "kf_fa_bwd": (
@@ -132,7 +138,7 @@ MEASURE_SIGNATURES = {
     "kfm_fa_fwd_split": (
         _int,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
-         _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _int, _int, _c_void_p],
+         _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _int, _int, _int, _int, _c_void_p],
     ),
     "kfm_fa_bwd_blocks": (
         _int,

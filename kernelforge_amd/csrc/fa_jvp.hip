@@ -122,18 +122,19 @@ template <int DP, int MODE> constexpr int fa_rows() { return FaTile<DP>::BQ * fa
 // first tO element of its first row (and nothing else), and fa_fixup_kernel
 // redoes its rows with LAZY = true, the scan that recomputes U.  kbuf0/1 and
 // vbuf0/1 are the two K-side and V-side LDS buffers, NT tiles each.  SPLIT
-// (FWD and FWD_JVP with LAZY = true): the workgroup scans one of p.splits key
-// ranges of its tile (fa_split_kernel).
-template <typename T, int DP, int MODE, bool ALL, bool LAZY, bool SPLIT = false>
+// (FWD and FWD_JVP with LAZY = true, JVP with LAZY = false): the workgroup scans
+// one of p.splits key ranges of its tile (fa_split_kernel).
+// DE <= DP: the head dim the products cover (LDS rows keep DP elements).
+template <typename T, int DP, int DE, int MODE, bool ALL, bool LAZY, bool SPLIT = false>
 __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T* vbuf0, T* vbuf1) {
-    static_assert(!SPLIT || (MODE != FA_JVP && LAZY), "the split scan is the rescaling one");
+    static_assert(!SPLIT || LAZY == (MODE != FA_JVP), "the split scan never needs a fixup for overflow");
     constexpr int R = SPLIT ? 1 : fa_row_blocks<DP, MODE>();
     constexpr int kBQ = FaTile<DP>::BQ * R, kBK = FaTile<DP>::BK;
     constexpr bool JVP = MODE != FA_FWD;
     constexpr bool kCachedO = MODE == FA_JVP && !LAZY;  // O from p.o, no U products
     constexpr int NT = JVP ? 2 : 1;   // tensors per side: K (, tK) and V (, tV)
-    constexpr int DS = DP / 32;        // 32-wide K-steps of the score products
-    constexpr int DB = DP / 16;        // 16-wide d blocks of the outputs
+    constexpr int DS = DE / 32;        // 32-wide K-steps of the score products
+    constexpr int DB = DE / 16;        // 16-wide d blocks of the outputs
     constexpr int NSTEP = 2 * DS;      // (key block, K-step) pairs of a half
     // Operand prefetch distance in MFMA steps; the forward has registers to
     // spare for a deeper ring.
@@ -221,8 +222,8 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
         }
     // The cached O values this lane's output elements need (d = 16*db +
     // 4*grp + 0..3; D % 8 == 0, so a chunk below D lies wholly below it).
-    typename V<T>::x4 ocv[R][kCachedO ? DB : 1];
-    if constexpr (kCachedO) {
+    typename V<T>::x4 ocv[R][kCachedO && !SPLIT ? DB : 1];
+    if constexpr (kCachedO && !SPLIT) {
 #pragma unroll
         for (int rb = 0; rb < R; ++rb)
 #pragma unroll
@@ -618,7 +619,7 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
         }
     }
 
-    if constexpr (kCachedO) {
+    if constexpr (kCachedO && !SPLIT) {
         // tO = G/l - (r/l) O with the cached O, unless a row's r/l could
         // amplify O's rounding past the bound: then only the marker is
         // written and fa_fixup_kernel redoes the workgroup's rows with U
@@ -664,8 +665,9 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
     }
 
     if constexpr (SPLIT) {
-        if (p.splits > 1) {
-            // The range's state; fa_combine_kernel joins the ranges.
+        if (MODE == FA_JVP || p.splits > 1) {
+            // The range's state; fa_combine_kernel (JVP: fa_combine_jvp_kernel)
+            // joins the ranges.
             const int64_t row = split * ((int64_t)p.B * p.Hq * p.Nq) + ((int64_t)b * p.Hq + row_head) * p.Nq + qr[0];
             const f32x4 st = {m_run[0], row_sum4(l_lse[0]), row_sum4(l_run[0]), row_sum4(r_run[0])};
             if (row_ok[0]) {
@@ -673,7 +675,7 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
                 for (int db = 0; db < DB; ++db) {
                     const int d = 16 * db + 4 * grp;
                     if (d < p.D) {
-                        *reinterpret_cast<f32x4*>(p.ws_u + row * p.D + d) = u[0][db];
+                        if constexpr (MODE != FA_JVP) *reinterpret_cast<f32x4*>(p.ws_u + row * p.D + d) = u[0][db];
                         if constexpr (JVP) *reinterpret_cast<f32x4*>(p.ws_g + row * p.D + d) = g[0][db];
                     }
                 }
@@ -727,12 +729,12 @@ __device__ __forceinline__ void fa_scan(const FaParams& p, T* kbuf0, T* kbuf1, T
     __shared__ __attribute__((aligned(16))) T vside0[NT_ * TILE_];         \
     __shared__ __attribute__((aligned(16))) T vside1[NT_ * TILE_]
 
-template <typename T, int DP, int MODE, bool ALL>
+template <typename T, int DP, int DE, int MODE, bool ALL>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
 void fa_kernel(const FaParams p) {
     FA_LDS_BUFFERS(T, DP, MODE);
-    fa_scan<T, DP, MODE, ALL, false>(p, kside0, kside1, vside0, vside1);
+    fa_scan<T, DP, DE, MODE, ALL, false>(p, kside0, kside1, vside0, vside1);
 }
 
 // Second launch of every mode: a workgroup whose rows carry the marker redoes
@@ -741,7 +743,7 @@ void fa_kernel(const FaParams p) {
 // first tO element of the workgroup's first row); every other workgroup reads
 // its markers and exits.  A separate kernel keeps that code out of the fast
 // scan's register allocation (inlined, the two scans spill at D = 128).
-template <typename T, int DP, int MODE, bool ALL>
+template <typename T, int DP, int DE, int MODE, bool ALL>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
 void fa_fixup_kernel(const FaParams p) {
@@ -759,7 +761,7 @@ void fa_fixup_kernel(const FaParams p) {
     }
     if (!__syncthreads_or(marked)) return;
     FA_LDS_BUFFERS(T, DP, MODE);
-    fa_scan<T, DP, MODE, ALL, true>(p, kside0, kside1, vside0, vside1);
+    fa_scan<T, DP, DE, MODE, ALL, true>(p, kside0, kside1, vside0, vside1);
 }
 
 // FWD and FWD_JVP for grids that would leave CUs idle: workgroups of one row
@@ -769,12 +771,12 @@ void fa_fixup_kernel(const FaParams p) {
 // workgroups.  The rescaling scan never overflows, so no fixup launch follows;
 // with one split the workgroup writes its results itself.  Both modes take the
 // same key ranges, so their LSE is the same sum.
-template <typename T, int DP, int MODE, bool ALL>
+template <typename T, int DP, int DE, int MODE, bool ALL>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
 void fa_split_kernel(const FaParams p) {
     FA_LDS_BUFFERS(T, DP, MODE);
-    fa_scan<T, DP, MODE, ALL, true, true>(p, kside0, kside1, vside0, vside1);
+    fa_scan<T, DP, DE, MODE, ALL, MODE != FA_JVP, true>(p, kside0, kside1, vside0, vside1);
 }
 
 // The results of each row from its key ranges' states (one wavefront per row),
@@ -836,7 +838,80 @@ __global__ __launch_bounds__(64 * kCombineRows) void fa_combine_kernel(const FaP
     if (lane == 0) p.lse[row] = empty ? __builtin_inff() : (m + log2f(l_lse)) * kLn2;
 }
 
-// How the forward modes cover a shape: splits = 0 is fa_kernel, otherwise
+// JVP: tO = G/l - (r/l) O of one 128-row (D > 128: 64-row) tile from its key
+// ranges' sums, four threads per row, with fa_kernel's bound on the cached O: a
+// tile past it gets the marker and fa_fixup_kernel redoes it.
+template <typename T, int DP>
+__global__ __launch_bounds__(FaTile<DP>::THREADS) void fa_combine_jvp_kernel(const FaParams p) {
+    static_assert(FaTile<DP>::THREADS == 4 * FaTile<DP>::BQ, "four threads per row");
+    constexpr int NV = DP / 16;  // float4 per thread
+    const FaBlock blk = fa_block(p);
+    const int iq = blk.qtile * FaTile<DP>::BQ + (int)(threadIdx.x >> 2), quarter = threadIdx.x & 3;
+    const bool ok = iq < p.Nq;
+    const int64_t rows = (int64_t)p.B * p.Hq * p.Nq;
+    const int64_t row = ((int64_t)blk.b * p.Hq + blk.hq) * p.Nq + (ok ? iq : 0);
+    const int64_t off = (((int64_t)blk.b * p.Nq + (ok ? iq : 0)) * p.Hq + blk.hq) * p.D;
+    const T* orow = static_cast<const T*>(p.o) + off;
+    T* torow = static_cast<T*>(p.to) + off;
+    float l = 0.f, r = 0.f;
+    f32x4 g[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) g[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Several ranges' loads in flight at a time (a range past the last re-reads
+    // it and is not added).
+    constexpr int UN = DP <= 128 ? 4 : 2;
+    for (int s0 = 0; s0 < p.splits; s0 += UN) {
+        f32x4 st[UN], v[UN][NV];
+#pragma unroll
+        for (int i = 0; i < UN; ++i) {
+            const int64_t at = min(s0 + i, p.splits - 1) * rows + row;
+            st[i] = reinterpret_cast<const f32x4*>(p.ws_st)[at];
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int d = 16 * j + 4 * quarter;
+                v[i][j] = *reinterpret_cast<const f32x4*>(p.ws_g + at * p.D + (d < p.D ? d : 0));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < UN; ++i)
+            if (s0 + i < p.splits) {
+                l += st[i][2];
+                r += st[i][3];
+#pragma unroll
+                for (int j = 0; j < NV; ++j) g[j] += v[i][j];
+            }
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f, rl = r * inv;
+    typename V<T>::x4 o[NV];
+    float om = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int d = 16 * j + 4 * quarter;
+        if (d < p.D) {
+            o[j] = *reinterpret_cast<const typename V<T>::x4*>(orow + d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) om = fmaxf(om, fabsf((float)o[j][e]));
+        }
+    }
+    om = fmaxf(om, __shfl_xor(om, 1, 64));
+    om = fmaxf(om, __shfl_xor(om, 2, 64));
+    if (__syncthreads_or(ok && fabsf(rl) * fmaxf(om, 1.f) > kCachedOBound)) {
+        if (threadIdx.x == 0) torow[0] = (T)__builtin_nanf("");
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int d = 16 * j + 4 * quarter;
+        if (ok && d < p.D) {
+            typename V<T>::x4 tv;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tv[e] = (T)(g[j][e] * inv - rl * (float)o[j][e]);
+            *reinterpret_cast<typename V<T>::x4*>(torow + d) = tv;
+        }
+    }
+}
+
+// How each mode covers a shape: splits = 0 is fa_kernel, otherwise
 // fa_split_kernel with that many key ranges per tile.
 struct FaSplitPlan {
     int splits, pack, n_qtiles;
@@ -859,14 +934,21 @@ constexpr int kMaxSplits = 64;  // one lane of fa_combine_kernel each
 //   B=1, N=2500, H=16/4, D=128, causal            71.3 -> 52.8 (1 range)
 // and where it keeps fa_kernel: B=4, N=1024, H=16, D=128 42.7 against 53.1
 // (1 range); B=2, N=2500, H=16/4, causal 78.0 against 81.9.
-FaSplitPlan fa_split_plan(const FaParams& p, int cus) {
+//
+// JVP: fa_kernel's tile already has the half size, and splitting keeps its
+// fixup launch; rows are not packed.  us: B=1, N=1000, H=8, D=128, causal 47.3 ->
+// 41.4 (4 ranges); B=1, N=700, H=4/2, D=256 51.8 -> 42.2 (3); B=1, N=1978, H=1,
+// D=128, causal 72 -> 41 (8).  At most 8 ranges: the join adds them one batch after
+// another per 128-row tile.
+FaSplitPlan fa_split_plan(const FaParams& p, int cus, int mode) {
+    const bool jvp = mode == FA_JVP;
     const int bq = p.D > 128 ? FaTile<256>::BQ : FaTile<128>::BQ;
     const int bk = p.D > 128 ? FaTile<256>::BK : FaTile<128>::BK;
-    const int full_rows = p.D > 128 ? fa_rows<256, FA_FWD>() : fa_rows<128, FA_FWD>();
+    const int full_rows = jvp ? bq : p.D > 128 ? fa_rows<256, FA_FWD>() : fa_rows<128, FA_FWD>();
     auto tiles = [](int64_t n, int64_t per) { return (n + per - 1) / per; };
     const int64_t flat = (int64_t)p.B * p.Hq * tiles(p.Nq, bq);
     const int64_t packed = (int64_t)p.B * p.Hkv * tiles((int64_t)p.group * p.Nq, bq);
-    FaSplitPlan plan{0, packed < flat ? 1 : 0, 0};
+    FaSplitPlan plan{0, !jvp && packed < flat ? 1 : 0, 0};
     const int64_t base = plan.pack ? packed : flat;
     plan.n_qtiles = (int)tiles(plan.pack ? (int64_t)p.group * p.Nq : p.Nq, bq);
     const int64_t ntiles = tiles(p.Nk, bk);
@@ -877,10 +959,11 @@ FaSplitPlan fa_split_plan(const FaParams& p, int cus) {
         return load > longest ? load : (double)longest;
     };
     double best = cost((int64_t)p.B * p.Hq * tiles(p.Nq, full_rows), ntiles) + 3.0;
-    const double half = p.D > 128 ? 1.35 : 0.8;
+    const double half = jvp ? 1.0 : p.D > 128 ? 1.35 : 0.8;
     const double traffic = (double)p.B * p.Hq * p.Nq * p.D * 8.0 / 7.8e6;
-    for (int s = 1; s <= kMaxSplits && (s == 1 || 2 * s <= ntiles) && (s == 1 || base * s <= 4 * (int64_t)cus); ++s) {
-        const double c = half * cost(base * s, tiles(ntiles, s)) + (s > 1 ? 5.0 + s * traffic : 0.0);
+    const int max_splits = jvp ? 8 : kMaxSplits;
+    for (int s = jvp ? 2 : 1; s <= max_splits && (s == 1 || 2 * s <= ntiles) && (s == 1 || base * s <= 4 * (int64_t)cus); ++s) {
+        const double c = half * cost(base * s, tiles(ntiles, s)) + (s > 1 ? 5.0 + s * traffic : 0.0) + (jvp ? 3.0 : 0.0);
         if (c < 0.95 * best) {  // clearly better than the plan with fewer workgroups
             best = c;
             plan.splits = s;
@@ -890,8 +973,26 @@ FaSplitPlan fa_split_plan(const FaParams& p, int cus) {
 }
 
 int64_t fa_split_ws_bytes(const FaParams& p, const FaSplitPlan& plan, int mode) {
-    if (plan.splits <= 1) return 0;
+    if (plan.splits <= (mode == FA_JVP ? 0 : 1)) return 0;
     return (int64_t)plan.splits * p.B * p.Hq * p.Nq * ((mode == FA_FWD_JVP ? 2 : 1) * p.D + 4) * (int64_t)sizeof(float);
+}
+
+// Padded head dims with a kernel; 96 keeps the LDS rows of 128 (B=2, N=4096,
+// H=16, D=72 on MI355X, us, padded to 128 and to 96: forward 236 and 214, fused
+// 632 and 555, JVP 564 and 497).
+int fa_pad_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : D <= 128 ? 128 : 256; }
+
+// Calls f(DP, DE) for a padded head dim.
+template <typename F> int fa_with_dims(int dp, F f) {
+    switch (dp) {
+        case 32: return f(std::integral_constant<int, 32>{}, std::integral_constant<int, 32>{});
+        case 64: return f(std::integral_constant<int, 64>{}, std::integral_constant<int, 64>{});
+        case 96: return f(std::integral_constant<int, 128>{}, std::integral_constant<int, 96>{});
+        case 128: return f(std::integral_constant<int, 128>{}, std::integral_constant<int, 128>{});
+        case 256: return f(std::integral_constant<int, 256>{}, std::integral_constant<int, 256>{});
+    }
+    set_error("fa: no kernel for padded head dim %d", dp);
+    return KF_E_UNSUPPORTED;
 }
 
 template <typename T, int MODE, bool ALL>
@@ -902,35 +1003,45 @@ int launch_split(FaParams p, const FaSplitPlan& plan, int dp, void* ws, hipStrea
     const int64_t rows = (int64_t)p.B * p.Hq * p.Nq;
     p.ws_st = static_cast<float*>(ws);
     p.ws_u = p.ws_st + (int64_t)p.splits * rows * 4;
-    p.ws_g = p.ws_u + (int64_t)p.splits * rows * p.D;
+    p.ws_g = MODE == FA_JVP ? p.ws_u : p.ws_u + (int64_t)p.splits * rows * p.D;
     const int64_t blocks = (int64_t)p.n_qtiles * (p.pack ? p.Hkv : p.Hq) * p.B * p.splits;
     if (blocks > 0x7fffffff) {
         set_error("fa: grid too large");
         return KF_E_UNSUPPORTED;
     }
-    auto launch = [&](auto dpc) {
-        constexpr int DP = decltype(dpc)::value;
-        hipLaunchKernelGGL((fa_split_kernel<T, DP, MODE, ALL>), dim3((unsigned)blocks), dim3(FaTile<DP>::THREADS), 0,
-                           stream, p);
-    };
-    switch (dp) {
-        case 32: launch(std::integral_constant<int, 32>{}); break;
-        case 64: launch(std::integral_constant<int, 64>{}); break;
-        case 128: launch(std::integral_constant<int, 128>{}); break;
-        default: launch(std::integral_constant<int, 256>{}); break;
-    }
-    if (int rc = check_launch("fa_split_kernel launch")) return rc;
-    if (p.splits == 1) return KF_OK;
-    hipLaunchKernelGGL((fa_combine_kernel<T, MODE>), dim3((unsigned)((rows + kCombineRows - 1) / kCombineRows)),
-                       dim3(64 * kCombineRows), 0, stream, p);
-    return check_launch("fa_combine_kernel launch");
+    return fa_with_dims(dp, [&](auto dpc, auto dec) {
+        constexpr int DP = decltype(dpc)::value, DE = decltype(dec)::value;
+        hipLaunchKernelGGL((fa_split_kernel<T, DP, DE, MODE, ALL>), dim3((unsigned)blocks),
+                           dim3(FaTile<DP>::THREADS), 0, stream, p);
+        if (int rc = check_launch("fa_split_kernel launch")) return rc;
+        if constexpr (MODE == FA_JVP) {
+            const dim3 tiles((unsigned)(blocks / p.splits));
+            hipLaunchKernelGGL((fa_combine_jvp_kernel<T, DP>), tiles, dim3(FaTile<DP>::THREADS), 0, stream, p);
+            if (int rc = check_launch("fa_combine_jvp_kernel launch")) return rc;
+            hipLaunchKernelGGL((fa_fixup_kernel<T, DP, DE, MODE, ALL>), tiles, dim3(FaTile<DP>::THREADS), 0, stream, p);
+            return check_launch("fa_fixup_kernel launch");
+        } else {
+            if (p.splits == 1) return (int)KF_OK;
+            hipLaunchKernelGGL((fa_combine_kernel<T, MODE>),
+                               dim3((unsigned)((rows + kCombineRows - 1) / kCombineRows)), dim3(64 * kCombineRows), 0,
+                               stream, p);
+            return check_launch("fa_combine_kernel launch");
+        }
+    });
 }
 
 template <typename T>
 int launch_split_mode(int mode, const FaParams& p, const FaSplitPlan& plan, int dp, void* ws, hipStream_t stream) {
-    if (mode == FA_FWD) return launch_split<T, FA_FWD, true>(p, plan, dp, ws, stream);
-    if (p.tq && p.tk && p.tv) return launch_split<T, FA_FWD_JVP, true>(p, plan, dp, ws, stream);
-    return launch_split<T, FA_FWD_JVP, false>(p, plan, dp, ws, stream);
+    const bool all = p.tq && p.tk && p.tv;
+    switch (mode) {
+        case FA_FWD: return launch_split<T, FA_FWD, true>(p, plan, dp, ws, stream);
+        case FA_FWD_JVP:
+            return all ? launch_split<T, FA_FWD_JVP, true>(p, plan, dp, ws, stream)
+                       : launch_split<T, FA_FWD_JVP, false>(p, plan, dp, ws, stream);
+        default:
+            return all ? launch_split<T, FA_JVP, true>(p, plan, dp, ws, stream)
+                       : launch_split<T, FA_JVP, false>(p, plan, dp, ws, stream);
+    }
 }
 
 template <typename T, int MODE, bool ALL>
@@ -941,21 +1052,13 @@ int launch_variant(const FaParams& p, int dp, hipStream_t stream) {
         return KF_E_UNSUPPORTED;
     }
     const dim3 grid((unsigned)blocks);
-    auto launch = [&](auto dpc) {
-        constexpr int DP = decltype(dpc)::value;
-        hipLaunchKernelGGL((fa_kernel<T, DP, MODE, ALL>), grid, dim3(FaTile<DP>::THREADS), 0, stream, p);
-        const int rc = check_launch("fa_kernel launch");
-        if (rc != KF_OK) return rc;
-        hipLaunchKernelGGL((fa_fixup_kernel<T, DP, MODE, ALL>), grid, dim3(FaTile<DP>::THREADS), 0, stream, p);
+    return fa_with_dims(dp, [&](auto dpc, auto dec) {
+        constexpr int DP = decltype(dpc)::value, DE = decltype(dec)::value;
+        hipLaunchKernelGGL((fa_kernel<T, DP, DE, MODE, ALL>), grid, dim3(FaTile<DP>::THREADS), 0, stream, p);
+        if (int rc = check_launch("fa_kernel launch")) return rc;
+        hipLaunchKernelGGL((fa_fixup_kernel<T, DP, DE, MODE, ALL>), grid, dim3(FaTile<DP>::THREADS), 0, stream, p);
         return check_launch("fa_fixup_kernel launch");
-    };
-    switch (dp) {
-        case 32: return launch(std::integral_constant<int, 32>{});
-        case 64: return launch(std::integral_constant<int, 64>{});
-        case 128: return launch(std::integral_constant<int, 128>{});
-        case 256: return launch(std::integral_constant<int, 256>{});
-        default: set_error("fa: head dim %d not supported by this build", p.D); return KF_E_UNSUPPORTED;
-    }
+    });
 }
 
 // The JVP modes have a branch-free instantiation for the common case of
@@ -982,7 +1085,7 @@ int fa_dispatch(int mode, FaParams p, int dtype, hipStream_t stream, void* ws = 
     if (p.B == 0 || p.Nq == 0) return KF_OK;
     KF_REQUIRE(p.q && p.k && p.v && p.o && p.lse && (mode == FA_FWD || p.to), KF_E_INVALID,
                "fa: null pointer");
-    const int dp = p.D <= 32 ? 32 : p.D <= 64 ? 64 : p.D <= 128 ? 128 : 256;
+    const int dp = fa_pad_dim(p.D);
     const int bq = dp > 128 ? fa_rows<256, FA_FWD_JVP>() : mode == FA_FWD ? fa_rows<128, FA_FWD>() : fa_rows<128, FA_FWD_JVP>();
     p.group = p.Hq / p.Hkv;
     p.n_qtiles = (p.Nq + bq - 1) / bq;
@@ -991,8 +1094,8 @@ int fa_dispatch(int mode, FaParams p, int dtype, hipStream_t stream, void* ws = 
         // No keys: O = 0 and tO = 0 by the empty-row convention; the kernel
         // handles it with zero tiles.
     }
-    if (mode != FA_JVP && p.Nk > 0) {
-        FaSplitPlan plan = forced ? *forced : fa_split_plan(p, device_cu_count());
+    if (p.Nk > 0) {
+        FaSplitPlan plan = forced ? *forced : fa_split_plan(p, device_cu_count(), mode);
         if (forced) {
             const int64_t rows = plan.pack ? (int64_t)p.group * p.Nq : p.Nq;
             const int tile = dp > 128 ? FaTile<256>::BQ : FaTile<128>::BQ;
@@ -1060,7 +1163,7 @@ int64_t fwd_workspace_bytes(int mode, int64_t B, int64_t Nq, int64_t Nk, int64_t
     FaParams p = make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, Nq,
                              Nk, Hq, Hkv, D, 1.f, causal);
     p.group = p.Hq / p.Hkv;
-    return fa_split_ws_bytes(p, fa_split_plan(p, device_cu_count()), mode);
+    return fa_split_ws_bytes(p, fa_split_plan(p, device_cu_count(), mode), mode);
 }
 }  // namespace
 }  // namespace kf
@@ -1086,6 +1189,23 @@ extern "C" int kf_fa_fwd_jvp_ws(const void* q, const void* k, const void* v, con
                        dtype, static_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 
+extern "C" int64_t kf_fa_jvp_workspace_bytes(int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv, int64_t D,
+                                             int causal) {
+    return kf::fwd_workspace_bytes(kf::FA_JVP, B, Nq, Nk, Hq, Hkv, D, causal);
+}
+
+extern "C" int kf_fa_jvp_ws(const void* q, const void* k, const void* v, const void* tq, const void* tk,
+                            const void* tv, const void* o, const float* lse, void* to, void* workspace,
+                            int64_t workspace_bytes, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
+                            int64_t D, float scale, int causal, int dtype, kf_stream_t stream) {
+    using namespace kf;
+    KF_REQUIRE(dims_fit(B, Nq, Nk, Hq, Hkv, D), KF_E_INVALID, "fa: shape out of range");
+    KF_REQUIRE((uintptr_t)workspace % 16 == 0, KF_E_WORKSPACE, "fa: workspace must be 16-byte aligned");
+    return fa_dispatch(FA_JVP, make_params(q, k, v, tq, tk, tv, const_cast<void*>(o), const_cast<float*>(lse), to, B,
+                                           Nq, Nk, Hq, Hkv, D, scale, causal),
+                       dtype, static_cast<hipStream_t>(stream), workspace, workspace_bytes);
+}
+
 extern "C" int kf_fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
                             int64_t workspace_bytes, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
                             int64_t D, float scale, int causal, int dtype, kf_stream_t stream) {
@@ -1098,20 +1218,22 @@ extern "C" int kf_fa_fwd_ws(const void* q, const void* k, const void* v, void* o
 }
 
 // Test entry point (not in the public header): kf_fa_fwd_ws, or kf_fa_fwd_jvp_ws
-// when `to` is not null, with the split kernels forced to `splits` key ranges
-// (0: fa_kernel) with packed rows or not.
+// when `to` is not null, or kf_fa_jvp_ws (cached != 0: o and lse are inputs),
+// with the split kernels forced to `splits` key ranges (0: fa_kernel) with
+// packed rows or not.
 extern "C" int kfm_fa_fwd_split(const void* q, const void* k, const void* v, const void* tq, const void* tk,
                                 const void* tv, void* o, float* lse, void* to, void* workspace,
                                 int64_t workspace_bytes, int64_t B, int64_t Nq, int64_t Nk, int64_t Hq, int64_t Hkv,
                                 int64_t D, float scale, int causal, int dtype, int splits, int pack,
-                                kf_stream_t stream) {
+                                int cached, kf_stream_t stream) {
     using namespace kf;
     KF_REQUIRE(dims_fit(B, Nq, Nk, Hq, Hkv, D) && Hkv > 0, KF_E_INVALID, "fa: shape out of range");
     KF_REQUIRE(splits >= 0 && splits <= kMaxSplits, KF_E_INVALID, "fa: splits must be 0..%d", kMaxSplits);
-    const int mode = to ? FA_FWD_JVP : FA_FWD;
+    const int mode = cached ? FA_JVP : to ? FA_FWD_JVP : FA_FWD;
     const FaParams p = make_params(q, k, v, tq, tk, tv, o, lse, to, B, Nq, Nk, Hq, Hkv, D, scale, causal);
     const FaSplitPlan forced{splits, pack ? 1 : 0, 0};
-    KF_REQUIRE(workspace_bytes >= fa_split_ws_bytes(p, forced, mode) && (splits <= 1 || workspace), KF_E_WORKSPACE,
+    KF_REQUIRE(workspace_bytes >= fa_split_ws_bytes(p, forced, mode) && (splits <= (cached ? 0 : 1) || workspace),
+               KF_E_WORKSPACE,
                "fa: split workspace too small");
     return fa_dispatch(mode, p, dtype, static_cast<hipStream_t>(stream), workspace, workspace_bytes, &forced);
 }

@@ -150,11 +150,12 @@ def _launch_jvp(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tq: torch.Ten
     q, k, v, out, lse = (x.contiguous() for x in (q, k, v, out, lse))
     B, Nq, Nk, Hq, Hkv, D = _dims(q, k)
     tout = torch.empty_like(out)
-    rc = _lib.load().kf_fa_jvp(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(tq), _lib.ptr(tk),
-                               _lib.ptr(tv), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(tout),
-                               B, Nq, Nk, Hq, Hkv, D, scale, int(causal), _lib.kf_dtype(q.dtype),
-                               _lib.stream_of(q))
-    _lib.check(rc, "kf_fa_jvp")
+    lib = _lib.load()
+    ws, ws_bytes = _split_workspace(lib.kf_fa_jvp_workspace_bytes(B, Nq, Nk, Hq, Hkv, D, int(causal)), q.device)
+    rc = lib.kf_fa_jvp_ws(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(tq), _lib.ptr(tk), _lib.ptr(tv),
+                          _lib.ptr(out), _lib.ptr(lse), _lib.ptr(tout), _lib.ptr(ws), ws_bytes,
+                          B, Nq, Nk, Hq, Hkv, D, scale, int(causal), _lib.kf_dtype(q.dtype), _lib.stream_of(q))
+    _lib.check(rc, "kf_fa_jvp_ws")
     return tout
 
 

@@ -25,16 +25,16 @@ def tensors(B, Nq, Nk, Hq, Hkv, D, dtype, seed=5):
                  for s in ((B, Nq, Hq, D), (B, Nk, Hkv, D), (B, Nk, Hkv, D)))
 
 
-def forced(q, k, v, causal, splits, pack, tangents=(None, None, None), jvp=False):
+def forced(q, k, v, causal, splits, pack, tangents=(None, None, None), jvp=False, cached=None):
     B, Nq, Hq, D = q.shape
     Nk, Hkv = k.shape[1:3]
-    out = torch.full_like(q, float("nan"))
-    lse = torch.full((B, Hq, Nq), float("nan"), device=DEV)
+    out, lse = cached or (torch.full_like(q, float("nan")), torch.full((B, Hq, Nq), float("nan"), device=DEV))
     to = torch.full_like(q, float("nan")) if jvp else None
     ws = torch.full((max(splits, 1) * B * Hq * Nq * (2 * D + 4),), float("nan"), device=DEV)
     rc = _lib.load().kfm_fa_fwd_split(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), *map(_lib.ptr, tangents),
                                       _lib.ptr(out), _lib.ptr(lse), _lib.ptr(to), _lib.ptr(ws), ws.numel() * 4, B, Nq, Nk, Hq, Hkv, D, D ** -0.5, int(causal),
-                                      _lib.kf_dtype(q.dtype), splits, int(pack), _lib.stream_of(q))
+                                      _lib.kf_dtype(q.dtype), splits, int(pack), int(cached is not None),
+                                      _lib.stream_of(q))
     _lib.check(rc, "kfm_fa_fwd_split")
     return (out, lse, to) if jvp else (out, lse)
 
@@ -66,6 +66,15 @@ def test_every_split(case, dtype):
         assert torch.equal(lse2, lse)
         torch.testing.assert_close(o2.cpu().double(), want, **BOUNDS[dtype])
         torch.testing.assert_close(to.cpu().double(), want_t, **BOUNDS[dtype])
+    # The JVP from cached results: one range is fa_kernel's own sum.
+    cached = forced(q, k, v, causal, 0, 0)
+    for splits in (0, 1, 2, 7, 64):
+        to = forced(q, k, v, causal, splits, 0, tangents, True, cached)[2]
+        torch.testing.assert_close(to.cpu().double(), want_t, **BOUNDS[dtype])
+        if splits == 0:
+            plain = to
+        if splits == 1:
+            assert torch.equal(to, plain)
     # Absent tangents are zeros.
     zero = torch.zeros_like(tangents[1])
     some = forced(q, k, v, causal, 3, 1, (tangents[0], None, tangents[2]), jvp=True)
@@ -88,6 +97,24 @@ def test_growing_scores_rescale(splits, pack):
     torch.testing.assert_close(out.cpu().double(), want, **BOUNDS[torch.bfloat16])
     torch.testing.assert_close(lse.cpu().double(), orc.attention_lse(q.cpu().double(), k.cpu().double()),
                                atol=1e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("splits", [0, 3])
+def test_jvp_peaked_tiles_recompute_the_output(splits):
+    """Tiles past the cached-O bound (a strongly peaked softmax) are redone with
+    O recomputed: the result does not depend on the cached out there, and does
+    on tiles under the bound."""
+    q, k, v = tensors(1, 256, 300, 2, 2, 64, torch.bfloat16)
+    tangents = tensors(1, 256, 300, 2, 2, 64, torch.bfloat16, seed=6)
+    q = q.clone()
+    q[:, 128:] *= 16  # the second 128-row tile is peaked
+    out, lse = forced(q, k, v, False, 0, 0)
+    plain = forced(q, k, v, False, splits, 0, tangents, True, (out, lse))[2]
+    moved = forced(q, k, v, False, splits, 0, tangents, True, (out + 0.25, lse))[2]
+    assert torch.equal(plain[:, 128:], moved[:, 128:])
+    assert not torch.equal(plain[:, :128], moved[:, :128])
+    _, want = orc.attention_jvp(*(t.cpu().double() for t in (q, k, v, *tangents)))
+    torch.testing.assert_close(plain.cpu().double(), want, **BOUNDS[torch.bfloat16])
 
 
 def test_nan_key_stays_in_its_head():
