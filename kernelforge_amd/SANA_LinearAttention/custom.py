@@ -32,6 +32,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+from functools import lru_cache
 
 import torch
 
@@ -61,9 +62,10 @@ def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int]) -
     fill of a fresh tensor would only run when the graph that happened to
     allocate it is replayed, while later graphs captured on the same stream
     share the tensor."""
-    stream = torch.cuda.current_stream(device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
-    capturing = torch.cuda.is_current_stream_capturing()
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    stream = _lib.current_stream(index)
+    key = (index, stream)
+    capturing = torch._C._cuda_isCurrentStreamCapturing()
     with _ws_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
@@ -74,7 +76,7 @@ def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int]) -
         lib = _lib.load()
         control = lib.kf_linattn_control_bytes(*shape)
         if control:
-            rc = lib.kf_linattn_workspace_init(_lib.ptr(ws), control, ctypes.c_void_p(stream.cuda_stream))
+            rc = lib.kf_linattn_workspace_init(_lib.ptr(ws), control, ctypes.c_void_p(stream))
             _lib.check(rc, "kf_linattn_workspace_init")
     return ws
 
@@ -99,8 +101,9 @@ def check_status(device: torch.device | int | None = None) -> None:
         _check_workspace(ws, ctypes.c_void_p(stream_handle))
 
 
-def _launch(kind: str, qkv: torch.Tensor, out: torch.Tensor, B: int, N: int, heads: int, dim: int, eps: float,
-            splits: int | None, check: bool) -> None:
+@lru_cache(maxsize=4096)
+def _sizes(device: torch.device, B: int, N: int, heads: int, dim: int, splits: int | None) -> tuple[int, int]:
+    """(splits, workspace bytes) of a call's shape on a device."""
     lib = _lib.load()
     if splits is None:
         splits = int(lib.kf_linattn_default_splits(B, heads, dim, N))
@@ -109,7 +112,13 @@ def _launch(kind: str, qkv: torch.Tensor, out: torch.Tensor, B: int, N: int, hea
     # The library runs at most one split per 32-token tile (its smallest split
     # unit), so a larger request needs no larger workspace.
     ws_splits = min(splits, max(1, -(-N // 32)))
-    ws_bytes = int(lib.kf_linattn_workspace_bytes(B, heads, dim, ws_splits))
+    return splits, int(lib.kf_linattn_workspace_bytes(B, heads, dim, ws_splits))
+
+
+def _launch(kind: str, qkv: torch.Tensor, out: torch.Tensor, B: int, N: int, heads: int, dim: int, eps: float,
+            splits: int | None, check: bool) -> None:
+    lib = _lib.load()
+    splits, ws_bytes = _sizes(qkv.device, B, N, heads, dim, splits)
     ws = _workspace(qkv.device, ws_bytes, (B, heads, dim))
     stream = _lib.stream_of(qkv)
     if kind == "fwd":

@@ -15,7 +15,7 @@ implement (flash-attention-jvp-derivation.md:388-558):
 - ``flash_attention_fwd_jvp(q, k, v, tq, tk, tv, *, softmax_scale, causal)``
   returning ``(out, lse, tangent)`` from one scan over the K/V tiles.
 
-Every operator is a ``torch.library.custom_op`` with a fake implementation,
+Every operator is registered with torch.library and has a fake implementation,
 so torch.func transforms unwrap their tensors before the C ABI sees raw
 pointers and torch.compile can trace them.  The standalone JVP is the
 reference's ``kernelforge::flash_attention_jvp`` (same schema,
@@ -32,6 +32,7 @@ heads of a GQA group summed in a fixed order, so gradients are deterministic.
 
 from __future__ import annotations
 
+import inspect
 import math
 
 import torch
@@ -111,8 +112,28 @@ def _split_workspace(nbytes: int, device: torch.device) -> tuple[torch.Tensor | 
 # ---------------------------------------------------------------------------
 # Opaque operators (C ABI launches on the current stream).
 # ---------------------------------------------------------------------------
-@torch.library.custom_op("kernelforge_amd::flash_attention_fwd", mutates_args=(), device_types="cuda")
-def _fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
+# Each forward operator is registered twice: as a custom_op under its public
+# name, and as a plain torch.library.Library operator (leading underscore) that
+# this module calls.  custom_op's Python autograd layer, which refuses a backward
+# through the operator, costs 10 us a call; the module's own calls never record
+# autograd (FlashAttentionFunction.forward and the no_grad
+# flash_attention_fwd_jvp make them) and do without it.
+_ops = torch.library.Library("kernelforge_amd", "FRAGMENT")
+
+
+def _register(schema: str, kernel, fake):
+    """Define ``kernelforge_amd::<schema>`` and ``kernelforge_amd::_<schema>`` with
+    a GPU kernel and a fake one; returns the second operator."""
+    name = schema.partition("(")[0]
+    torch.library.custom_op(f"kernelforge_amd::{name}", kernel, mutates_args=(), device_types="cuda",
+                            schema=schema[len(name):]).register_fake(fake)
+    _ops.define("_" + schema, tags=(torch.Tag.pt2_compliant_tag,))
+    _ops.impl("_" + name, kernel, "CUDA")
+    torch.library.register_fake(f"kernelforge_amd::_{name}", fake, lib=_ops)
+    return getattr(torch.ops.kernelforge_amd, "_" + name).default
+
+
+def _fwd_kernel(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
             causal: bool) -> tuple[torch.Tensor, torch.Tensor]:
     B, Nq, Nk, Hq, Hkv, D = _dims(q, k)
     out = torch.empty_like(q)
@@ -126,9 +147,12 @@ def _fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
     return out, lse
 
 
-@_fwd_op.register_fake
 def _fwd_fake(q, k, v, scale, causal):
     return torch.empty_like(q), q.new_empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32)
+
+
+_fwd_op = _register("flash_attention_fwd(Tensor q, Tensor k, Tensor v, float scale, bool causal) -> (Tensor, Tensor)",
+                    _fwd_kernel, _fwd_fake)
 
 
 @torch.library.custom_op("kernelforge::flash_attention_jvp", mutates_args=(), device_types="cuda")
@@ -164,8 +188,7 @@ def _launch_jvp_fake(q, k, v, tq, tk, tv, out, lse, scale, causal, block_m, bloc
     return torch.empty_like(out)
 
 
-@torch.library.custom_op("kernelforge_amd::flash_attention_fwd_jvp", mutates_args=(), device_types="cuda")
-def _fwd_jvp_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tq: torch.Tensor | None,
+def _fwd_jvp_kernel(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tq: torch.Tensor | None,
                 tk: torch.Tensor | None, tv: torch.Tensor | None, scale: float,
                 causal: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     B, Nq, Nk, Hq, Hkv, D = _dims(q, k)
@@ -181,10 +204,13 @@ def _fwd_jvp_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tq: torch.Ten
     return out, lse, tout
 
 
-@_fwd_jvp_op.register_fake
 def _fwd_jvp_fake(q, k, v, tq, tk, tv, scale, causal):
     lse = q.new_empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32)
     return torch.empty_like(q), lse, torch.empty_like(q)
+
+
+_fwd_jvp_op = _register("flash_attention_fwd_jvp(Tensor q, Tensor k, Tensor v, Tensor? tq, Tensor? tk, Tensor? tv, "
+                        "float scale, bool causal) -> (Tensor, Tensor, Tensor)", _fwd_jvp_kernel, _fwd_jvp_fake)
 
 
 @torch.library.custom_op("kernelforge_amd::flash_attention_bwd", mutates_args=(), device_types="cuda")
@@ -328,6 +354,11 @@ class FlashAttentionFunction(torch.autograd.Function):
         tangent = flash_attention_jvp(q, k, v, tq, tk, tv, out, lse,
                                       softmax_scale=ctx.softmax_scale, causal=ctx.causal)
         return tangent, None
+
+
+# Function.apply binds its arguments through inspect.signature(forward) on every
+# call (8 us); a stored signature is returned as it is.
+FlashAttentionFunction.forward.__signature__ = inspect.signature(FlashAttentionFunction.forward)
 
 
 def flash_attention(q, k, v, *, softmax_scale=None, causal=False, return_lse=False):
