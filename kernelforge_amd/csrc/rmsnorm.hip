@@ -427,7 +427,9 @@ __global__ __launch_bounds__(64 * WAVES) void rmsnorm_bwd_vec_kernel(const TX* _
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int j = (i * WPR + slice) * 64 + lane;
-        wv[i] = reinterpret_cast<const WPack*>(w)[j < nvec ? j : 0];
+        // Zero past the row's end, as x and dy are (another column's weight
+        // may be infinite, and its product with zero would be NaN).
+        wv[i] = j < nvec ? reinterpret_cast<const WPack*>(w)[j] : WPack{};
 #pragma unroll
         for (int k = 0; k < VEC; ++k) acc[i][k] = 0.f;
     }

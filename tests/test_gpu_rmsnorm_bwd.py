@@ -80,3 +80,14 @@ def test_infinite_row_stays_in_its_row():
     keep[[5, 17]] = False
     assert torch.equal(dx[keep], clean[keep])
     assert bool(torch.isnan(dx[5]).any()) and bool(torch.isnan(dx[17]).all())
+
+
+@pytest.mark.parametrize("dim", [8, 504, 1032, 2240, 4104])
+def test_infinite_weight(dim):
+    """An infinite weight makes its own column's dx infinite or NaN and the other
+    columns' infinite, also where the row leaves vectors of a wavefront unused."""
+    x = (1 + torch.rand(3, dim, device=DEV)).to(BF16)
+    w = torch.ones(dim, device=DEV)
+    w[0] = float("inf")
+    dx, dw = grads(x, w, torch.ones(3, dim, device=DEV))
+    assert bool(torch.isinf(dx[:, 1:]).all()) and bool(torch.isfinite(dw).all())
