@@ -231,6 +231,25 @@ int kf_linattn_attn_matmul(const void* qkv, float* out, void* workspace,
 int kf_linattn_check(void* workspace, int64_t workspace_bytes, kf_stream_t stream);
 
 /*
+ * kf_linattn_workspace_init for a workspace that is memory of a graph, recorded
+ * before the captured call of this shape (it does nothing for shapes and types
+ * without cross-workgroup counters).  Every replay then starts from zero
+ * control words, so the workspace need not outlive the capture.  It also makes
+ * the call report an incomplete result to a word of the device that replays
+ * leave alone: kf_linattn_capture_check reads it.
+ */
+int kf_linattn_capture_init(void* workspace, int64_t workspace_bytes, int64_t batch, int64_t heads, int64_t dim,
+                            int in_dtype, kf_stream_t stream);
+
+/*
+ * Status of the replayed launches prepared by kf_linattn_capture_init on the
+ * current device since the last check: waits for `stream`, returns KF_OK or
+ * KF_E_INCOMPLETE as kf_linattn_check does, and clears the word.  It reports
+ * every replay that has finished (synchronise the streams they ran on first).
+ */
+int kf_linattn_capture_check(kf_stream_t stream);
+
+/*
  * Largest scratch, in bytes, that kf_linattn_fwd_noalloc can use: the size
  * of its static device array (16 MiB), which must hold
  * kf_linattn_workspace_bytes(batch, heads, dim, splits).

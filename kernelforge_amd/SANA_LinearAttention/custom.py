@@ -51,12 +51,13 @@ def default_splits(batch: int, heads: int, dim: int, seq_len: int) -> int:
 
 _ws_lock = threading.Lock()
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
+_captured_devices: set[int] = set()  # devices some call was captured on
 
 
-def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int]) -> torch.Tensor:
+def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int, int]) -> torch.Tensor:
     """The zero-initialised workspace of the current stream on `device`, at
     least `nbytes` long (its control words are zero between calls); ``shape``
-    is the call's (batch, heads, dim).
+    is the call's (batch, heads, dim, input dtype code).
 
     Under graph capture the zeroing is recorded with every call instead: the
     fill of a fresh tensor would only run when the graph that happened to
@@ -73,11 +74,9 @@ def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int]) -
             ws = make(max(nbytes, 1 << 20), device=device, dtype=torch.uint8)
             _workspaces[key] = ws
     if capturing:
-        lib = _lib.load()
-        control = lib.kf_linattn_control_bytes(*shape)
-        if control:
-            rc = lib.kf_linattn_workspace_init(_lib.ptr(ws), control, ctypes.c_void_p(stream))
-            _lib.check(rc, "kf_linattn_workspace_init")
+        _captured_devices.add(index)
+        rc = _lib.load().kf_linattn_capture_init(_lib.ptr(ws), ws.numel(), *shape, ctypes.c_void_p(stream))
+        _lib.check(rc, "kf_linattn_capture_init")
     return ws
 
 
@@ -90,13 +89,19 @@ def check_status(device: torch.device | int | None = None) -> None:
     """Raise RuntimeError if a linear-attention launch on ``device`` since the
     last check gave up waiting for its split workgroups (its outputs are NaN).
 
-    Synchronises each stream that owns a workspace on the device; not for use
-    under graph capture.  Clears the condition it reports.
+    Synchronises each stream that owns a workspace on the device, and the whole
+    device once a call has been captured on it (replays report to a word of the
+    device); not for use under graph capture.  Clears the condition it reports.
     """
     dev = torch.device("cuda", device) if isinstance(device, int) else torch.device(device or "cuda")
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     with _ws_lock:
         items = [(key, ws) for key, ws in _workspaces.items() if key[0] == index]
+    if index in _captured_devices:
+        with torch.cuda.device(index):
+            torch.cuda.synchronize()
+            rc = _lib.load().kf_linattn_capture_check(ctypes.c_void_p(_lib.current_stream(index)))
+        _lib.check(rc, "kf_linattn_capture_check")
     for (_, stream_handle), ws in items:
         _check_workspace(ws, ctypes.c_void_p(stream_handle))
 
@@ -119,7 +124,7 @@ def _launch(kind: str, qkv: torch.Tensor, out: torch.Tensor, B: int, N: int, hea
             splits: int | None, check: bool) -> None:
     lib = _lib.load()
     splits, ws_bytes = _sizes(qkv.device, B, N, heads, dim, splits)
-    ws = _workspace(qkv.device, ws_bytes, (B, heads, dim))
+    ws = _workspace(qkv.device, ws_bytes, (B, heads, dim, _lib.kf_dtype(qkv.dtype)))
     stream = _lib.stream_of(qkv)
     if kind == "fwd":
         rc = lib.kf_linattn_fwd(_lib.ptr(qkv), _lib.ptr(out), _lib.ptr(ws), ws.numel(), B, N, heads, dim,

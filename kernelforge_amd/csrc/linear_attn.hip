@@ -52,6 +52,8 @@ constexpr int kSpinLimit = 1 << 20; // polls of the group counter before giving 
 //   [1]          error word: 1 = a group barrier timed out, 2 = control words
 //                not zero on entry (a ticket beyond the grid, or a group
 //                counter above its member count)
+//   [2]          kReportToDevice = errors also go to the device's
+//                `captured_error` word (kf_linattn_capture_init)
 //   [64 + 64g]   arrivals of group g (one (batch, head pair)) at its barrier
 //   [64 + 64g+1] departures of group g from it (each group's words share no
 //                cache line with another group's, so polls do not collide)
@@ -64,6 +66,19 @@ constexpr int kCtrlStride = 64;            // words per group: each group's coun
 constexpr int kMaxGroupsPerLaunch = 4096;  // larger problems take several launches
 constexpr int64_t kCtrlBytes = (int64_t)(kCtrlHeader + kCtrlStride * kMaxGroupsPerLaunch) * 4;
 static_assert(kCtrlBytes % 256 == 0, "partials stay 256-byte aligned");
+
+// Error word of the launches recorded into graphs, whose workspaces are graph
+// memory: their own error words are cleared by every replay, and the memory
+// may hold something else between replays.  Written only by a launch that
+// gives up; one per device, zero at load.
+static __device__ unsigned captured_error;
+constexpr unsigned kReportToDevice = 0x4b464345u;  // not what dirty control words are likely to hold
+
+__device__ __forceinline__ void report_error(unsigned* ctrl, unsigned code) {
+    __hip_atomic_store(ctrl + 1, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_load(ctrl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kReportToDevice)
+        __hip_atomic_store(&captured_error, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Workgroup barrier that leaves global loads in flight.  __syncthreads()
 // also waits for every outstanding global load (vmcnt(0)), which would drain
@@ -209,7 +224,7 @@ __device__ __forceinline__ bool group_barrier(unsigned* ctrl, int g, unsigned me
         unsigned seen;
         while ((seen = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < members) {
             if (++polls > spin_limit) {
-                __hip_atomic_store(ctrl + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                report_error(ctrl, 1u);
                 late = 1;
                 break;
             }
@@ -225,7 +240,7 @@ __device__ __forceinline__ bool group_barrier(unsigned* ctrl, int g, unsigned me
         // words were not zero on entry.  Reported like a stale ticket; the
         // partials may be incomplete, so this member writes NaN.
         if (seen > members || departed >= members) {
-            __hip_atomic_store(ctrl + 1, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            report_error(ctrl, 2u);
             late = 1;
         }
         *late_flag = late;
@@ -319,7 +334,7 @@ __global__ __launch_bounds__(kThreads) void linattn_fused_kernel(FusedParams p) 
         if (ticket >= p.total) {
             // Control words that were not zero on entry: flag it and touch
             // nothing (the group barriers of the other workgroups then time out).
-            if (tid == 0) __hip_atomic_store(p.ctrl + 1, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (tid == 0) report_error(p.ctrl, 2u);
             return;
         }
     }
@@ -694,8 +709,9 @@ int launch_reduce(const float* partial, float* state, int64_t n_heads, int split
 }
 
 // Zeroes n words (the control words of a fresh workspace).
-__global__ __launch_bounds__(256) void linattn_zero_kernel(unsigned* __restrict__ p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0u;
+__global__ __launch_bounds__(256) void linattn_zero_kernel(unsigned* __restrict__ p, int64_t n, unsigned word2) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        p[i] = i == 2 ? word2 : 0u;
 }
 
 // --------------------------------------------------------------------------
@@ -1037,13 +1053,15 @@ int64_t resolve_splits(int64_t batch, int64_t seq_len, int64_t heads, int64_t di
     return eff;
 }
 
-// Zeroes the first `bytes` of a workspace (rounded down to whole words).
-int zero_words(void* ws, int64_t bytes, hipStream_t s) {
+// Zeroes the first `bytes` of a workspace (rounded down to whole words), its
+// word 2 set to `word2` instead.
+int zero_words(void* ws, int64_t bytes, hipStream_t s, unsigned word2 = 0u) {
     const int64_t n = bytes / 4;
     if (n <= 0) return KF_OK;
     int64_t blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(linattn_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<unsigned*>(ws), n);
+    hipLaunchKernelGGL(linattn_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<unsigned*>(ws), n,
+                       word2);
     return check_launch("linattn_zero_kernel launch");
 }
 
@@ -1120,16 +1138,15 @@ int scratch_for_current_device(void** ptr, hipStream_t stream) {
     return KF_OK;
 }
 
-// Reads the error word of a control region after `stream` has drained; when
-// it is set, clears the whole control region (a ticket counter may be left
-// over too) and reports what happened.
-int check_ctrl(unsigned* ctrl, hipStream_t stream) {
+// Reads an error word after `stream` has drained; when it is set, clears
+// `bytes` at `region`, which holds it, and reports what happened.
+int check_word(const unsigned* error, unsigned* region, int64_t bytes, hipStream_t stream) {
     unsigned word = 0;
-    hipError_t err = hipMemcpyAsync(&word, ctrl + 1, sizeof(word), hipMemcpyDeviceToHost, stream);
+    hipError_t err = hipMemcpyAsync(&word, error, sizeof(word), hipMemcpyDeviceToHost, stream);
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
     if (err != hipSuccess) return hip_failure(err, "linattn check: reading the error word");
     if (word == 0) return KF_OK;
-    if (int rc = zero_words(ctrl, kCtrlBytes, stream)) return rc;
+    if (int rc = zero_words(region, bytes, stream)) return rc;
     err = hipStreamSynchronize(stream);
     if (err != hipSuccess) return hip_failure(err, "linattn check: clearing the control words");
     if (word == 1)
@@ -1140,6 +1157,10 @@ int check_ctrl(unsigned* ctrl, hipStream_t stream) {
                   "outputs are incomplete", word);
     return KF_E_INCOMPLETE;
 }
+
+// A control region's error word; a set one clears the whole region (a ticket
+// counter may be left over too).
+int check_ctrl(unsigned* ctrl, hipStream_t stream) { return check_word(ctrl + 1, ctrl, kCtrlBytes, stream); }
 
 // Validates, then runs kf_linattn_fwd's request on the static scratch.
 int noalloc_run(const void* qkv, void* out, int64_t batch, int64_t seq_len, int64_t heads, int64_t dim,
@@ -1214,6 +1235,16 @@ extern "C" int kf_linattn_workspace_init(void* workspace, int64_t workspace_byte
     return zero_words(workspace, n, static_cast<hipStream_t>(stream));
 }
 
+extern "C" int kf_linattn_capture_init(void* workspace, int64_t workspace_bytes, int64_t batch, int64_t heads,
+                                       int64_t dim, int in_dtype, kf_stream_t stream) {
+    using namespace kf;
+    const int64_t n = fused_candidate(dim, in_dtype) ? kf_linattn_control_bytes(batch, heads, dim) : 0;
+    if (n == 0) return KF_OK;
+    KF_REQUIRE(workspace && workspace_bytes >= n, KF_E_WORKSPACE,
+               "linattn: %lld bytes of control words needed, %lld given", (long long)n, (long long)workspace_bytes);
+    return zero_words(workspace, n, static_cast<hipStream_t>(stream), kReportToDevice);
+}
+
 extern "C" int kf_linattn_fwd(const void* qkv, void* out, void* workspace, int64_t workspace_bytes,
                               int64_t batch, int64_t seq_len, int64_t heads, int64_t dim,
                               int64_t splits, float eps, int in_dtype, int out_dtype,
@@ -1240,6 +1271,15 @@ extern "C" int kf_linattn_check(void* workspace, int64_t workspace_bytes, kf_str
     KF_REQUIRE(workspace && workspace_bytes >= kCtrlBytes, KF_E_WORKSPACE,
                "linattn check: a workspace of at least %lld bytes is needed", (long long)kCtrlBytes);
     return check_ctrl(static_cast<unsigned*>(workspace), static_cast<hipStream_t>(stream));
+}
+
+extern "C" int kf_linattn_capture_check(kf_stream_t stream) {
+    using namespace kf;
+    void* word = nullptr;
+    const hipError_t err = hipGetSymbolAddress(&word, HIP_SYMBOL(captured_error));
+    if (err != hipSuccess) return hip_failure(err, "linattn: hipGetSymbolAddress(captured_error)");
+    return check_word(static_cast<unsigned*>(word), static_cast<unsigned*>(word), sizeof(unsigned),
+                      static_cast<hipStream_t>(stream));
 }
 
 extern "C" int64_t kf_linattn_noalloc_max_bytes(void) { return kLinattnScratchBytes; }
