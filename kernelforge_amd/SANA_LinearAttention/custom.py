@@ -13,7 +13,7 @@ a counter, sums their partials in a fixed order (deterministic) and
 contracts the state with relu(q) on MFMA, all in one launch.  The counters
 and partials live in a workspace kept per (device, stream): allocated zeroed
 once, grown when a call needs more, and left with zero counters by every
-call.
+call.  A captured call's workspace is memory of its graph instead.
 
 ``attn_matmul(q, k, v, eps)`` is ``LiteLA.attn_matmul`` itself (original.py:
 99-117) on the same kernel: q ``[B, h, d, N]``, k ``[B, h, N, d]``, v ``[B, h,
@@ -59,24 +59,26 @@ def _workspace(device: torch.device, nbytes: int, shape: tuple[int, int, int, in
     least `nbytes` long (its control words are zero between calls); ``shape``
     is the call's (batch, heads, dim, input dtype code).
 
-    Under graph capture the zeroing is recorded with every call instead: the
-    fill of a fresh tensor would only run when the graph that happened to
-    allocate it is replayed, while later graphs captured on the same stream
-    share the tensor."""
+    Under graph capture every call has a workspace of its own from the graph's
+    memory, cleared by a recorded launch: a workspace of the table may be
+    replaced while the graph still points to it, would be shared by graphs
+    replayed on different streams, and one made under capture holds nothing an
+    eager call could rely on."""
     index = device.index if device.index is not None else torch.cuda.current_device()
     stream = _lib.current_stream(index)
+    nbytes = max(nbytes, 1 << 20)
+    if torch._C._cuda_isCurrentStreamCapturing():
+        ws = torch.empty(nbytes, device=device, dtype=torch.uint8)
+        _captured_devices.add(index)
+        rc = _lib.load().kf_linattn_capture_init(_lib.ptr(ws), nbytes, *shape, ctypes.c_void_p(stream))
+        _lib.check(rc, "kf_linattn_capture_init")
+        return ws
     key = (index, stream)
-    capturing = torch._C._cuda_isCurrentStreamCapturing()
     with _ws_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
-            make = torch.empty if capturing else torch.zeros
-            ws = make(max(nbytes, 1 << 20), device=device, dtype=torch.uint8)
+            ws = torch.zeros(nbytes, device=device, dtype=torch.uint8)
             _workspaces[key] = ws
-    if capturing:
-        _captured_devices.add(index)
-        rc = _lib.load().kf_linattn_capture_init(_lib.ptr(ws), ws.numel(), *shape, ctypes.c_void_p(stream))
-        _lib.check(rc, "kf_linattn_capture_init")
     return ws
 
 

@@ -1,5 +1,5 @@
 """Linear-attention calls recorded into graphs: what check_status() reports of
-their replays."""
+their replays, and that graphs and eager calls never meet in a workspace."""
 
 import pytest
 import torch
@@ -63,3 +63,73 @@ def test_check_status_reports_an_earlier_node(monkeypatch):
         check_status()
     assert reported, "no member stopped waiting at a two-poll limit"
     assert torch.equal(linear_attention(qkv, 4, 32, splits=8, check=True), want)
+
+
+def capture(stream, *calls):
+    """A graph of linear_attention calls on ``stream``, whose pool first held a
+    tensor of nonzero bytes."""
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        junk = torch.full((32 << 20,), 1, dtype=torch.uint8, device=DEV)
+        del junk
+        outs = [linear_attention(qkv, H, D) for qkv, H, D in calls]
+    return graph, outs
+
+
+def test_eager_call_on_the_capture_stream():
+    """An eager call on the stream of a capture, with more (batch, head pair)
+    groups than the captured calls cleared, before and after replays."""
+    small, other = packed(1, 300, 4, 32, seed=2), packed(1, 300, 3, 64, seed=3)
+    big = packed(2, 512, 36, 32, seed=4)
+    want = [linear_attention(x, H, D) for x, H, D in ((small, 4, 32), (other, 3, 64), (big, 36, 32))]
+    check_status()
+    stream = torch.cuda.Stream()
+    for first, D in (((other, 3, 64), 64), ((small, 4, 32), 32)):
+        print(f"captured D={D}", flush=True)
+        graph, outs = capture(stream, first)
+        for replays in (0, 1, 2):
+            with torch.cuda.stream(stream):
+                for _ in range(replays):
+                    graph.replay()
+                got = linear_attention(big, 36, 32)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want[2])
+            check_status()
+        assert torch.equal(outs[0], want[1] if D == 64 else want[0])
+
+
+def test_graphs_keep_their_workspaces():
+    """Replays after a larger eager call on the capture stream and tensors in
+    the memory it may have freed, after another graph of the stream is gone,
+    and of two graphs at once on two streams."""
+    a, b = packed(1, 2048, 8, 32, seed=5), packed(2, 1500, 24, 32, seed=6)
+    large = packed(2, 4096, 70, 32, seed=7)
+    want_a, want_b = linear_attention(a, 8, 32), linear_attention(b, 24, 32)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        linear_attention(a, 8, 32)
+    gone, _ = capture(stream, (a, 8, 32))
+    ga, (out_a,) = capture(stream, (a, 8, 32))
+    gb, (out_b,) = capture(stream, (b, 24, 32))
+    with torch.cuda.stream(stream):
+        linear_attention(large, 70, 32)
+    del gone
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    filler = [torch.full((1 << 20,), 3, dtype=torch.uint8, device=DEV) for _ in range(64)]
+    other = torch.cuda.Stream()
+    for rep in range(4):
+        print(f"replay {rep}", flush=True)
+        out_a.fill_(float("nan"))
+        out_b.fill_(float("nan"))
+        stream.wait_stream(torch.cuda.current_stream())
+        other.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            ga.replay()
+        with torch.cuda.stream(other):
+            gb.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out_a, want_a) and torch.equal(out_b, want_b)
+        assert all(bool((f == 3).all()) for f in filler)
+        check_status()

@@ -1,5 +1,5 @@
-"""Two captured LiteLA blocks whose graphs share the capture stream's
-linear-attention workspace: either may be replayed first, and often."""
+"""Two LiteLA blocks captured on one stream, a workspace of its own for each
+captured call: either graph may be replayed first, and often."""
 
 import pytest
 import torch
