@@ -17,7 +17,8 @@ This is the general-shape form of the reference's fused
 which exist there for one shape only.
 
 Head dim 32, bf16 or fp16.  The partials live in a workspace kept per
-(device, stream) and grown when a call needs more.
+(device, stream) and grown when a call needs more; a captured call's is memory
+of its graph.
 
 ``prefer_fused`` is the modules' choice between this path and the unfused one
 (projection GEMM, then the linear-attention kernel).  The fused tiles are tied
@@ -50,6 +51,13 @@ _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
+    """The current stream's workspace on `device`, at least `nbytes` long (it
+    needs no initialisation).  Under graph capture every call has one of its
+    own from the graph's memory: a graph would keep pointing to a workspace of
+    the table after growth replaced it, and share it with graphs replayed on
+    other streams."""
+    if torch._C._cuda_isCurrentStreamCapturing():
+        return torch.empty(nbytes, device=device, dtype=torch.uint8)
     index = device.index if device.index is not None else torch.cuda.current_device()
     key = (index, _lib.current_stream(index))
     with _ws_lock:

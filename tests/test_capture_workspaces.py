@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from kernelforge_amd import _lib
-from kernelforge_amd.SANA_LinearAttention import custom
+from kernelforge_amd.SANA_LinearAttention import custom, fused
 
 CPU = torch.device("cpu", 0)
 
@@ -58,3 +58,17 @@ def test_linear_attention_workspaces(device, monkeypatch):
     again = custom._workspace(CPU, 1 << 20, shape)
     assert again.data_ptr() not in (eager.data_ptr(), captured.data_ptr())
     assert list(custom._workspaces.values()) == [eager]
+
+
+def test_fused_projection_workspaces(device, monkeypatch):
+    monkeypatch.setattr(fused, "_workspaces", {})
+    capturing, _ = device
+    capturing(True)
+    captured = fused._workspace(CPU, 4096)
+    assert captured.numel() >= 4096 and not fused._workspaces
+    capturing(False)
+    eager = fused._workspace(CPU, 8192)
+    assert fused._workspace(CPU, 4096) is eager
+    capturing(True)
+    assert fused._workspace(CPU, 4096).data_ptr() not in (eager.data_ptr(), captured.data_ptr())
+    assert list(fused._workspaces.values()) == [eager]

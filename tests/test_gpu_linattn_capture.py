@@ -6,6 +6,7 @@ import torch
 
 from kernelforge_amd import _lib
 from kernelforge_amd.SANA_LinearAttention import check_status, custom, linear_attention
+from kernelforge_amd.SANA_LinearAttention.fused import litela_fused_attention
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -133,3 +134,43 @@ def test_graphs_keep_their_workspaces():
         assert torch.equal(out_a, want_a) and torch.equal(out_b, want_b)
         assert all(bool((f == 3).all()) for f in filler)
         check_status()
+
+
+def test_fused_projection_graphs_on_two_streams():
+    """Graphs of the fused projection path captured on one stream and replayed
+    at once on two, after a larger eager call on the capture stream."""
+    def inputs(B, N, H, seed):
+        g = torch.Generator().manual_seed(seed)
+        x = torch.randn((B, N, 32 * H), generator=g)
+        w = torch.randn((96 * H, 32 * H), generator=g) * (32 * H) ** -0.5
+        return x.to(torch.bfloat16).to(DEV), w.to(torch.bfloat16).to(DEV), H
+
+    def run(x, w, H):
+        return litela_fused_attention(x, w, None, H)
+
+    cases = [inputs(1, 700, 12, 1), inputs(2, 900, 9, 2)]
+    large = inputs(2, 2048, 36, 3)
+    want = [run(*c) for c in cases]
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        run(*cases[0])
+    graphs, outs = [], []
+    for case in cases:
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=stream):
+            outs.append(run(*case))
+    with torch.cuda.stream(stream):
+        run(*large)
+    torch.cuda.synchronize()
+    streams = [stream, torch.cuda.Stream()]
+    for rep in range(4):
+        print(f"replay {rep}", flush=True)
+        for out in outs:
+            out.fill_(float("nan"))
+        for s, graph in zip(streams, graphs):
+            s.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(s):
+                graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(out, w) for out, w in zip(outs, want))
