@@ -108,8 +108,10 @@ def _norm_rotate_(qkv: torch.Tensor, heads: int, dim: int, q_norm_weight, k_norm
     cos, sin = tables if tables is not None else (None, None)
     if q_norm_weight is not None:
         qw, kw = (w.detach().to(qkv.dtype).contiguous() for w in (q_norm_weight, k_norm_weight))
+        _lib.require_gpu(qkv, qw, kw)
         row_bytes = C * qkv.element_size()
-        one_pass = (0 < row_bytes <= 16384 and row_bytes % 16 == 0 and qw.numel() == kw.numel() == C
+        # Weights of another shape are refused by rms_norm_rows_.
+        one_pass = (0 < row_bytes <= 16384 and row_bytes % 16 == 0 and qw.shape == kw.shape == (C,)
                     and (cos is None or dim % 8 == 0)
                     and all(t is None or t.data_ptr() % 16 == 0 for t in (qkv, qw, kw, cos, sin)))
         if one_pass:
