@@ -225,8 +225,13 @@ def current_stream(device_index: int) -> int:
 
 
 def stream_of(t: torch.Tensor) -> ctypes.c_void_p:
-    """hipStream_t of torch's current stream on t's device."""
-    return ctypes.c_void_p(current_stream(t.get_device()))
+    """hipStream_t of torch's current stream on t's device.  A tensor that is on
+    no GPU is refused: for its device index, -1, torch returns the current
+    device's stream, and the launch would take a host pointer."""
+    index = t.get_device()
+    if index < 0:
+        require_gpu(t)
+    return ctypes.c_void_p(current_stream(index))
 
 
 def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
