@@ -184,8 +184,9 @@ template <typename T, int VPT, int WPR, int WAVES, int ROPE>
 __global__ __launch_bounds__(64 * WAVES) void rmsnorm_qk_kernel(T* qkv, const T* __restrict__ qw,
                                                                 const T* __restrict__ kw,
                                                                 const float* __restrict__ cs,
-                                                                const float* __restrict__ sn, int64_t tokens,
-                                                                int64_t N, int dim, int D, float eps) {
+                                                                const float* __restrict__ sn, int64_t row0,
+                                                                int64_t tokens, int64_t N, int dim, int D,
+                                                                float eps) {
     // The rotary products and their sum are rounded one by one (rope.hip).
 #pragma clang fp contract(off)
     constexpr int VEC = 16 / sizeof(T);
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(64 * WAVES) void rmsnorm_qk_kernel(T* qkv, const T*
     constexpr int RPB = WAVES / WPR;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int slot = wave / WPR, slice = wave % WPR;
-    const int64_t r = (int64_t)blockIdx.x * RPB + slot;  // a token's q row, then its k row
+    const int64_t r = row0 + (int64_t)blockIdx.x * RPB + slot;  // a token's q row, then its k row
     const int64_t tok = r >> 1;
     const int part_k = (int)(r & 1);
     const bool ok = tok < tokens;
@@ -271,18 +272,24 @@ __global__ __launch_bounds__(64 * WAVES) void rmsnorm_qk_kernel(T* qkv, const T*
 template <typename T, int VPT, int WPR, int WAVES>
 int launch_qk(void* qkv, const void* qw, const void* kw, const float* cs, const float* sn, int64_t tokens, int64_t N,
               int64_t dim, int64_t D, float eps, hipStream_t stream) {
-    const int64_t blocks = (2 * tokens + WAVES / WPR - 1) / (WAVES / WPR);
-    KF_REQUIRE(blocks <= 0x7fffff, KF_E_UNSUPPORTED, "qk_norm: %lld tokens exceed the grid limit", (long long)tokens);
-    const dim3 grid((unsigned)blocks);
-    auto launch = [&](auto ropec) {
-        hipLaunchKernelGGL((rmsnorm_qk_kernel<T, VPT, WPR, WAVES, decltype(ropec)::value>), grid, dim3(64 * WAVES), 0,
-                           stream, static_cast<T*>(qkv), static_cast<const T*>(qw), static_cast<const T*>(kw), cs, sn,
-                           tokens, N, (int)dim, (int)D, eps);
-    };
-    if (!cs) launch(std::integral_constant<int, 0>{});
-    else if (64 * (16 / (int)sizeof(T)) % D == 0) launch(std::integral_constant<int, 1>{});
-    else launch(std::integral_constant<int, 2>{});
-    return check_launch("rmsnorm_qk_kernel launch");
+    // Rows per launch: HIP limits a grid to 2^32 - 1 threads.  The two row
+    // norms this stands for took twice the tokens in one launch each.
+    constexpr int RPB = WAVES / WPR;
+    constexpr int64_t kMaxBlocks = 0xffffffffLL / (64 * WAVES);
+    for (int64_t row0 = 0; row0 < 2 * tokens; row0 += kMaxBlocks * RPB) {
+        const int64_t left = (2 * tokens - row0 + RPB - 1) / RPB;
+        const dim3 grid((unsigned)(left < kMaxBlocks ? left : kMaxBlocks));
+        auto launch = [&](auto ropec) {
+            hipLaunchKernelGGL((rmsnorm_qk_kernel<T, VPT, WPR, WAVES, decltype(ropec)::value>), grid,
+                               dim3(64 * WAVES), 0, stream, static_cast<T*>(qkv), static_cast<const T*>(qw),
+                               static_cast<const T*>(kw), cs, sn, row0, tokens, N, (int)dim, (int)D, eps);
+        };
+        if (!cs) launch(std::integral_constant<int, 0>{});
+        else if (64 * (16 / (int)sizeof(T)) % D == 0) launch(std::integral_constant<int, 1>{});
+        else launch(std::integral_constant<int, 2>{});
+        if (int rc = check_launch("rmsnorm_qk_kernel launch")) return rc;
+    }
+    return KF_OK;
 }
 
 template <typename T>

@@ -50,3 +50,26 @@ def test_refuses_what_it_does_not_cover():
     assert lib.kf_qk_norm_rope(*args, 1, 1, 3, 4, 1e-5, bf, _lib.stream_of(t)) != 0      # 24-byte rows
     assert lib.kf_qk_norm_rope(*args, 1, 1, 512, 32, 1e-5, bf, _lib.stream_of(t)) != 0   # over 16 KiB
     assert lib.kf_qk_norm_rope(_lib.ptr(t[..., 1:]), *args[1:], 1, 1, 2, 32, 1e-5, bf, _lib.stream_of(t)) != 0
+
+
+@pytest.mark.parametrize("rope", [False, True])
+def test_more_rows_than_one_launch_takes(rope):
+    """33.6 million tokens: 67.1 million rows of q and k, four to a workgroup of
+    256 threads, pass the 2^32 - 1 threads of one grid inside a sequence."""
+    B, N, D = 5, 6_711_000, 8
+    assert 2 * B * N * 64 > 2 ** 32 - 1
+    g = torch.Generator(DEV).manual_seed(3)
+    got = torch.empty(B, N, 3, D, device=DEV, dtype=torch.bfloat16).normal_(generator=g)
+    qw, kw = (torch.empty(D, device=DEV, dtype=torch.bfloat16).normal_(1, 0.1, generator=g) for _ in range(2))
+    angle = torch.empty(N, D, device=DEV).uniform_(0, 6, generator=g)
+    cos, sin = angle.cos(), angle.sin()
+    want = got.clone()
+    rms_norm_rows_(want[:, :, 0], qw, 1e-5)
+    rms_norm_rows_(want[:, :, 1], kw, 1e-5)
+    lib, bf, stream = _lib.load(), _lib.KF_BF16, _lib.stream_of(got)
+    if rope:
+        _lib.check(lib.kf_rope_packed(*map(_lib.ptr, (want, cos, sin)), B, N, 1, D, bf, stream), "kf_rope_packed")
+    tables = (cos, sin) if rope else (None, None)
+    _lib.check(lib.kf_qk_norm_rope(*map(_lib.ptr, (got, qw, kw, *tables)), B, N, 1, D, 1e-5, bf, stream),
+               "kf_qk_norm_rope")
+    assert torch.equal(got, want)
