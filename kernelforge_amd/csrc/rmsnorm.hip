@@ -616,11 +616,11 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const TX* __restric
 constexpr int kDwCols = 32, kDwSlices = 16;
 template <typename TW>
 __global__ __launch_bounds__(kDwCols * kDwSlices) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial,
-                                                                                 TW* __restrict__ dw, int64_t dim,
-                                                                                 int nblocks) {
+                                                                                 TW* __restrict__ dw, int64_t c0,
+                                                                                 int64_t dim, int nblocks) {
     __shared__ float sums[kDwSlices][kDwCols];
     const int col = threadIdx.x % kDwCols, slice = threadIdx.x / kDwCols;
-    const int64_t c = (int64_t)blockIdx.x * kDwCols + col;
+    const int64_t c = c0 + (int64_t)blockIdx.x * kDwCols + col;
     float acc = 0.f;
     if (c < dim) {
         for (int b0 = slice; b0 < nblocks; b0 += 8 * kDwSlices) {
@@ -708,9 +708,16 @@ int run_bwd(const void* x, const void* w, const void* dy, void* dx, void* dw, fl
             return rc;
     }
     // With no rows the reduction adds nothing and writes a zero weight gradient.
-    hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<TW>), dim3((unsigned)((dim + kDwCols - 1) / kDwCols)),
-                       dim3(kDwCols * kDwSlices), 0, stream, partial, static_cast<TW*>(dw), dim, (int)used);
-    return check_launch("rmsnorm_dw_reduce_kernel launch");
+    // Sixteen threads a column: HIP's limit of 2^32 - 1 threads in a grid is
+    // passed at 2^28 columns.
+    constexpr int64_t kMaxBlocks = 0xffffffffLL / (kDwCols * kDwSlices);
+    for (int64_t c0 = 0; c0 < dim; c0 += kMaxBlocks * kDwCols) {
+        const int64_t left = (dim - c0 + kDwCols - 1) / kDwCols;
+        hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<TW>), dim3((unsigned)(left < kMaxBlocks ? left : kMaxBlocks)),
+                           dim3(kDwCols * kDwSlices), 0, stream, partial, static_cast<TW*>(dw), c0, dim, (int)used);
+        if (int rc = check_launch("rmsnorm_dw_reduce_kernel launch")) return rc;
+    }
+    return KF_OK;
 }
 
 bool valid_dt(int d) { return d == KF_F32 || d == KF_F16 || d == KF_BF16; }

@@ -12,6 +12,7 @@ sum of those half ulps.
 import pytest
 import torch
 
+from kernelforge_amd import _lib
 from kernelforge_amd.rmsnorm.custom import rms_norm_module_forward
 
 pytestmark = pytest.mark.gpu
@@ -91,3 +92,22 @@ def test_infinite_weight(dim):
     w[0] = float("inf")
     dx, dw = grads(x, w, torch.ones(3, dim, device=DEV))
     assert bool(torch.isinf(dx[:, 1:]).all()) and bool(torch.isfinite(dw).all())
+
+
+@pytest.mark.parametrize("rows", [0, 1])
+def test_more_columns_than_one_reduction_launch_takes(rows):
+    """2^28 columns at 16 threads each pass the 2^32 - 1 threads of one grid.
+    Entries of +-1 have a mean square of 1 (their sums are exact), so dw is dy
+    with x's signs; with no rows it is zero."""
+    dim = 2 ** 28 + 40
+    g = torch.Generator(DEV).manual_seed(rows)
+    signs = torch.empty(rows, dim, device=DEV, dtype=BF16).bernoulli_(0.5, generator=g) * 2 - 1
+    dy = torch.empty(rows, dim, device=DEV, dtype=BF16).normal_(generator=g)
+    w = torch.ones(dim, device=DEV, dtype=BF16)
+    dx, dw = torch.empty_like(signs), torch.full_like(w, float("nan"))
+    lib = _lib.load()
+    nbytes = lib.kf_rmsnorm_bwd_workspace_bytes(rows, dim)
+    ws = torch.empty(nbytes, device=DEV, dtype=torch.uint8)
+    _lib.check(lib.kf_rmsnorm_bwd(*map(_lib.ptr, (signs, w, dy, dx, dw, ws)), nbytes, rows, dim, 1e-6, _lib.KF_BF16,
+                                  _lib.KF_BF16, _lib.stream_of(w)), "kf_rmsnorm_bwd")
+    assert torch.equal(dw, (signs * dy)[0] if rows else torch.zeros_like(w))
