@@ -143,6 +143,7 @@ template <typename T, int BN, bool KN> struct ProjTile {
 template <typename T> struct Tile64x64 { typedef GemmCfg<T, 64, 64, 4, 4, false> C; };
 template <typename T> struct Tile128x64 { typedef GemmCfg<T, 128, 64, 4, 3, false> C; };
 template <typename T> struct Tile128x128 { typedef GemmCfg<T, 128, 128, 2, 2, false> C; };
+static_assert(Tile64x64<bf16>::C::THREADS == 512, "pick_tile's grid limit");
 
 template <typename C>
 int launch_cfg(GemmParams p, bool bias, hipStream_t stream) {
@@ -196,6 +197,9 @@ inline int pick_tile(int M, int N) {
     static const Small small[] = {{64, 64, 0.32, 0.46}, {128, 64, 0.40, 0.70}, {128, 128, 0.61, 1.02}};
     for (int i = 0; i < 3; ++i) {
         const long long n = (long long)((M + small[i].bm - 1) / small[i].bm) * ((N + small[i].bn - 1) / small[i].bn);
+        // HIP limits a grid to 2^32 - 1 threads (512 a workgroup); the 256-row
+        // tiles reach further (narrow outputs of over 2^29 rows).
+        if (n > 0xffffffffLL / 512) continue;
         const long long rest = n % (2 * cus);
         const double cost = (double)(n / (2 * cus)) * small[i].c2 + (rest == 0 ? 0 : rest <= cus ? small[i].c1 : small[i].c2);
         if (cost < best_cost) {

@@ -41,3 +41,16 @@ def test_tiles_agree(M, N, K, dtype, bias):
     exact = (xi.double() @ wi.double().T + (bi.double() if bias else 0)).to(dtype)
     for tile in (1, 2, 3):
         assert torch.equal(run(xi.to(DEV), wi.to(DEV), bi.to(DEV) if bias else None, tile).cpu(), exact), tile
+
+
+def test_more_rows_than_a_small_tile_grid_takes():
+    """537 million rows of 8 columns: 64-row tiles of 512 threads pass the
+    2^32 - 1 threads of one grid, the 256-row tiles do not."""
+    M, K, N = 2 ** 29 + 100, 8, 8
+    g = torch.Generator(DEV).manual_seed(1)
+    x = torch.empty(M, K, device=DEV, dtype=torch.bfloat16).random_(-3, 4, generator=g)
+    w = torch.empty(N, K, device=DEV, dtype=torch.bfloat16).random_(-3, 4, generator=g)
+    y = linear(x, w)
+    for r0 in (0, M // 2, M - 5000):
+        rows = x[r0:r0 + 5000].cpu().double()
+        assert torch.equal(y[r0:r0 + 5000].cpu(), (rows @ w.cpu().double().T).to(torch.bfloat16))
