@@ -298,7 +298,7 @@ void linattn_wide_out_kernel(const T* __restrict__ qkv, const float* __restrict_
     constexpr int QM = QC < 16 ? QC - 1 : 15, OM = OC < 16 ? OC - 1 : 15;
     __shared__ __attribute__((aligned(16))) unsigned char qt[TT * QC * 16];
     __shared__ __attribute__((aligned(16))) unsigned char ot[OT ? 16 : TT * OC * 16];
-    __shared__ float inv_den[TT * HG];
+    __shared__ float2 inv_den[TT * HG];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = blockIdx.x;
@@ -395,7 +395,15 @@ void linattn_wide_out_kernel(const T* __restrict__ qkv, const float* __restrict_
             }
 #pragma unroll
             for (int off = 1; off < LPH; off <<= 1) d += __shfl_xor(d, off, 64);
-            if (lch % LPH == 0) inv_den[tok * HG + lch / LPH] = 1.0f / (d + eps);
+            if (lch % LPH == 0) {
+                // 1 / den as a product of two factors, the second 1 unless den
+                // is under 2^-124 or over 2^124: its reciprocal alone could be
+                // infinite or subnormal where the quotient is neither.
+                const float den = d + eps;
+                const float mag = fabsf(den);
+                const float up = mag < 0x1p-124f ? 0x1p64f : mag > 0x1p124f ? 0x1p-64f : 1.f;
+                inv_den[tok * HG + lch / LPH] = make_float2(1.0f / (den * up), up);
+            }
         }
     };
     auto contract = [&](int t0) {
@@ -423,20 +431,20 @@ void linattn_wide_out_kernel(const T* __restrict__ qkv, const float* __restrict_
                         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sf[k][e], q[e], acc, 0, 0, 0);
                 }
             }
-            const float inv = inv_den[tok * HG + hh];
+            const float2 inv = inv_den[tok * HG + hh];
             const int r = r0 + 4 * (lane >> 4);  // this lane's rows r..r+3
             if constexpr (OT) {
                 if (head_ok && t0 + tok < t_end) {
                     float* dst = reinterpret_cast<float*>(out) + ((int64_t)b * C + (int64_t)(h0 + hh) * D + r) * N +
                                  t0 + tok;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) __builtin_nontemporal_store(acc[e] * inv, dst + (int64_t)e * N);
+                    for (int e = 0; e < 4; ++e) __builtin_nontemporal_store(acc[e] * inv.x * inv.y, dst + (int64_t)e * N);
                 }
             } else {
                 typedef TO out4 __attribute__((ext_vector_type(4)));
                 out4 o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = from_f32<TO>(acc[e] * inv);
+                for (int e = 0; e < 4; ++e) o[e] = from_f32<TO>(acc[e] * inv.x * inv.y);
                 const int off = (hh * D + r) * (int)sizeof(TO);
                 *reinterpret_cast<out4*>(ot + (tok * OC + ((off >> 4) ^ (tok & OM))) * 16 + (off & 15)) = o;
             }

@@ -98,3 +98,24 @@ def test_special_values_stay_in_their_heads(dtype, D):
     fine = torch.isfinite(valu)
     assert rel(got[fine], valu[fine]) <= 2 * BOUND[torch.float32]
     assert torch.equal(got[..., 3 * D:], linear_attention(clean, H, D)[..., 3 * D:])
+
+
+# Denominators whose reciprocal overflows or is subnormal, with quotients near 1:
+# q and k are scaled so that z . relu(q), whose mean is 150 D E[relu^]^2 scale^2
+# = 24 D scale^2 for normal values, is about 1e-41 or 1.2e38 (fp32 ends at
+# 3.4e38).  A sum of 150 D terms of which each is rounded to a step of 2^-149 is
+# off by 2^-150 sqrt(150 D) at most typically, 1e-2 of 1e-41 at D = 128; the
+# large case loses nothing.
+@pytest.mark.parametrize("den,bound", [(1e-41, 1e-2), (1.2e38, BOUND[torch.float32])])
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 16), (torch.float32, 32), (torch.float32, 64),
+                                     (torch.float32, 128), (torch.bfloat16, 64), (torch.bfloat16, 128)])
+def test_denominators_at_the_ends_of_the_range(dtype, D, den, bound):
+    B, N, H = 1, 150, 3
+    qkv = packed(B, N, H, D, torch.float32, seed=D)
+    qkv[:, :, :2] *= (den / (24 * D)) ** 0.5
+    qkv = qkv.to(dtype)
+    want = exact(qkv, H, D, eps=0.0)
+    got = linear_attention(qkv.to(DEV), H, D, eps=0.0)
+    assert bool(torch.isfinite(got).all())
+    assert rel(got.cpu(), want) <= bound
+    assert rel(linear_attention(unaligned(qkv.to(DEV)), H, D, eps=0.0).cpu(), want) <= bound
