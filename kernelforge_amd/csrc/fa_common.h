@@ -94,11 +94,11 @@ struct FaParams {
     float scale;       // natural units
     float scale_log2;  // scale * log2(e)
     int causal;
-    // Split forward modes (fa_split_kernel) only.
+    // fa_split_kernel and its joins only.
     int splits;        // key ranges per query tile
     int pack;          // rows of a tile: 1 = (query, head of the KV head's group) pairs, 0 = queries of one head
-    float* ws_u;       // [splits][B * Hq * Nq][D] unnormalised outputs U (splits > 1)
-    float* ws_g;       // the same of G (FWD_JVP)
+    float* ws_u;       // [splits][B * Hq * Nq][D] unnormalised outputs U (FWD, FWD_JVP; splits > 1)
+    float* ws_g;       // the same of G (FWD_JVP; JVP at any split count)
     float* ws_st;      // [splits][B * Hq * Nq][4]: exponent reference (log2), fp32 row sum, l, r
 };
 

@@ -50,7 +50,8 @@
 // the scan.  A later score exceeding m by ~2^7 (log2 units; 2^4 for fp16 E)
 // overflows to a non-finite accumulator, which the workgroup detects at the
 // end and answers by redoing its rows with a lazily rescaling scan (an
-// out-of-line function).  The JVP-from-LSE mode uses -LSE as the reference.
+// out-of-line function).  The split kernel's FWD/FWD_JVP scan rescales from the
+// start.  The JVP-from-LSE mode uses -LSE as the reference.
 #include "fa_common.h"
 
 namespace kf {
@@ -76,7 +77,7 @@ __device__ __forceinline__ FaBlock fa_block(const FaParams& p) {
     return r;
 }
 
-// The split forward's workgroup: a query tile, a head (KV head when rows are
+// The split kernel's workgroup: a query tile, a head (KV head when rows are
 // packed), a batch and a key range.  Tiles of one key range follow one another
 // (they share its K and V in an XCD's L2); under a causal mask every head's
 // longest tile starts before any shorter one instead.
@@ -764,13 +765,19 @@ void fa_fixup_kernel(const FaParams p) {
     fa_scan<T, DP, DE, MODE, ALL, true>(p, kside0, kside1, vside0, vside1);
 }
 
-// FWD and FWD_JVP for grids that would leave CUs idle: workgroups of one row
-// block per wavefront (in the forward half of fa_kernel's rows), the heads of a
-// KV group packed into one tile when that takes fewer tiles (decoding: K and V
-// are then read once per KV head), and the keys of a tile split over p.splits
-// workgroups.  The rescaling scan never overflows, so no fixup launch follows;
-// with one split the workgroup writes its results itself.  Both modes take the
-// same key ranges, so their LSE is the same sum.
+// Grids that would leave CUs idle: workgroups of one row block per wavefront (in
+// the forward half of fa_kernel's rows) and the keys of a tile split over
+// p.splits workgroups.  FWD and FWD_JVP also pack the heads of a KV group into
+// one tile when that takes fewer tiles (decoding: K and V are then read once per
+// KV head); their rescaling scan never overflows, so no fixup launch follows,
+// and with one split the workgroup writes its results itself.  JVP keeps
+// fa_kernel's scan (-LSE as the reference, the cached O), the join's bound test
+// and the fixup launch.
+//
+// FWD and FWD_JVP take the same key ranges, so their LSE is the same sum where
+// there are two or more.  With one, FWD_JVP runs fa_kernel: the sums are equal
+// bit for bit while no score passes the reference by the rescale threshold, and
+// beyond it differ by the rounding of exponents taken from two references.
 template <typename T, int DP, int DE, int MODE, bool ALL>
 __global__ __launch_bounds__(FaTile<DP>::THREADS)
 __attribute__((amdgpu_waves_per_eu(FaTile<DP>::OCC, FaTile<DP>::OCC)))
@@ -1069,7 +1076,7 @@ int launch_mode(const FaParams& p, int dp, hipStream_t stream) {
     return launch_variant<T, MODE, false>(p, dp, stream);
 }
 
-// ws / ws_bytes: the split forward's workspace (FWD, FWD_JVP); a call that was
+// ws / ws_bytes: the split kernel's workspace (every mode); a call that was
 // given none where its plan needs one runs fa_kernel.  forced: a plan's splits
 // and pack instead of the shape's own (n_qtiles is filled in).
 int fa_dispatch(int mode, FaParams p, int dtype, hipStream_t stream, void* ws = nullptr, int64_t ws_bytes = 0,

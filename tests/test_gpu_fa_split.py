@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from kernelforge_amd import _lib
-from kernelforge_amd.flash_attention_jvp import flash_attention
+from kernelforge_amd.flash_attention_jvp import flash_attention, flash_attention_fwd_jvp
 from oracle import fa as orc
 
 pytestmark = pytest.mark.gpu
@@ -124,3 +124,31 @@ def test_nan_key_stays_in_its_head():
     out = forced(q, k, v, False, 4, 1)[0]
     assert torch.equal(out[:, :, :2], clean[:, :, :2])
     assert bool(torch.isnan(out[:, :, 2:]).all()) == bool(torch.isnan(forced(q, k, v, False, 0, 0)[0][:, :, 2:]).all())
+
+
+# Scores that rise far past the first keys' maximum, without overflow (2^128 over
+# it in bf16, 2^16 in fp16).
+@pytest.mark.parametrize("dtype,growth,ref", [(torch.bfloat16, 10, 128), (torch.float16, 1.5, 16)])
+@pytest.mark.parametrize("shape", [(1, 333, 333, 16, 16, 64), (1, 700, 700, 16, 16, 128)])
+def test_one_range_lse_of_both_modes(shape, dtype, growth, ref):
+    """With one key range the forward rescales and the fused mode keeps its first
+    reference.  Exponents of up to ``ref`` log2 units from it carry half an ulp of
+    ref, which the sum, its log2 and the product with ln 2 each add once more at
+    most (scores here stay under 128 log2 units): 4 * 2^-17 * ln 2 in the worse mode,
+    twice that between the two."""
+    q, k, v = tensors(*shape, dtype)
+    k = (k * torch.linspace(0.1, growth, shape[2], device=DEV)[None, :, None, None]).to(dtype)
+    tangents = tensors(*shape, dtype, seed=6)
+    out, lse = flash_attention(q, k, v, return_lse=True)
+    out2, lse2, tangent = flash_attention_fwd_jvp(q, k, v, *tangents)
+    want, want_t = orc.attention_jvp(*(t.cpu().double() for t in (q, k, v, *tangents)))
+    lse_want = orc.attention_lse(q.cpu().double(), k.cpu().double())
+    scores = torch.einsum("bqhd,bkhd->bhqk", q.cpu().double(), k.cpu().double()) * shape[-1] ** -0.5 * 1.4427
+    rise = (scores.amax(-1) - scores[..., :32].amax(-1)).amax()
+    assert 8 < float(rise) < ref and float(scores.abs().max()) < 128
+    bound = 8 * 2.0 ** -17 * 0.6932
+    for got, exact in ((lse, lse_want), (lse2, lse_want), (lse, lse2)):
+        torch.testing.assert_close(got.cpu().double(), exact.cpu().double(), atol=bound, rtol=0)
+    for got, exact in ((out, want), (out2, want), (tangent, want_t)):
+        scale = max(1.0, float(exact.abs().max()))
+        torch.testing.assert_close(got.cpu().double() / scale, exact / scale, **BOUNDS[dtype])
