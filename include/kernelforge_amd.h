@@ -182,16 +182,17 @@ int64_t kf_linattn_control_bytes(int64_t batch, int64_t heads, int64_t dim);
  *
  * qkv: [batch, seq_len, 3, heads*dim] of in_dtype (KF_BF16 or KF_F16, or KF_F32);
  * out: [batch, seq_len, heads*dim] of out_dtype (KF_F32, KF_F16 or KF_BF16).
- * dim must be 32 for the MFMA kernel in this build (one launch: the split
- * workgroups of a (batch, head pair) meet at a counter in the workspace's
- * control words); other head dims and fp32 input take a three-launch VALU
- * path.  splits <= 0 selects kf_linattn_default_splits; any positive count is
+ * 16-bit input at dim 32 runs in one launch (the split workgroups of a
+ * (batch, head pair) meet at a counter in the workspace's control words).
+ * Other head dims from 16 and fp32 input take three launches on the matrix
+ * cores; dims 1..8, and qkv or out that are not 16-byte aligned, three on the
+ * VALU.  splits <= 0 selects kf_linattn_default_splits; any positive count is
  * accepted and used as an upper bound: it is cut to the sequence length and,
  * for the fused kernel, to the number of its workgroups the device holds at
  * once (occupancy per CU x CUs: 256 on MI355X for fp32 output), because a
  * group's split workgroups wait for each other and must be resident
- * together.  Each split then takes whole 128-token tiles (32 on the VALU
- * path), so fewer splits than requested may run.
+ * together.  Each split then takes whole 128-token tiles (32 on the other
+ * paths), so fewer splits than requested may run.
  * workspace: at least kf_linattn_workspace_bytes bytes for the requested
  * splits, 256-byte aligned, control words zero on entry
  * (kf_linattn_workspace_init); they are zero again on return.  The split

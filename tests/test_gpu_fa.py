@@ -126,7 +126,7 @@ def test_fused_single_pass(case, dtype):
                                atol=1e-3, rtol=1e-4)
     # The forward kernel divides by the fp32 sum of E, the fused one by the
     # sum of the 16-bit E its products use: O within two ulps, LSE (the same
-    # fp32 sum) bit for bit.
+    # fp32 sum, no score rising past the rescale threshold here) bit for bit.
     out_fwd, lse_fwd = flash_attention(q, k, v, return_lse=True, **opts(case))
     torch.testing.assert_close(out.float(), out_fwd.float(), atol=1e-6, rtol=2 * torch.finfo(dtype).eps)
     assert torch.equal(lse, lse_fwd)
